@@ -1,0 +1,139 @@
+// activation_split.h -- the activation halves of the exact batched products
+// (prefill_exact.hip, few_rows.hip).
+#pragma once
+
+#include "common.h"
+#include "block_reduce.h"
+#include "exact_blocks.h"
+
+#pragma clang fp contract(off)
+
+namespace holo {
+
+// ---- the activation halves: Ah, Al [M][K] f16, block sums Sx [M][K/32], row scales Rs [M] ----
+// One workgroup per row.  The row's values y (x; silu(g) * u as
+// cuda_silu_mul computes it, cuda_ops.cu:304-314; or the RMS-normed row,
+// rms_norm_rows4_k's arithmetic: thread t sums the squares of float4s
+// t + 256 j, the same workgroup reduction, x * scale * w, so the normed
+// values are the bits the separate norm writes) are scaled by a power of two
+// 2^e chosen from the row's largest magnitude a: a * 2^e lies in
+// [2^14, 2^15).  The halves then never overflow f16 (|y| up to fp32's range
+// is taken) and the low half is a normal f16 for every value above
+// a * 2^-17, so x - xh - xl stays within 2^-22 |x| there and within
+// a * 2^-40 below.  The product's store multiplies by Rs = 2^-e (exact).  A
+// 32-block is the 8 float4 of 8 adjacent lanes (K % 32 == 0); Sx holds the
+// block sums of the scaled values (for the Q4_K min term).
+// OPS: the halves in the operand order of few_rows.hip instead, and Sx as
+// [rows / 16][block][16]; n_zero counters at `zero` are cleared.  There the
+// low half of an infinite value is zero, so that the products of a row with
+// infinities are the infinities (and NaNs) that fp32 gives.
+namespace {
+enum XSplitMode { XS_PLAIN = 0, XS_SWIGLU = 1, XS_NORM = 2 };
+
+template <int NV, int MODE, int NT = 256, bool OPS = false>
+__global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2 *__restrict__ Al,
+                                                    float *__restrict__ Sx, float *__restrict__ Rs,
+                                                    const float *__restrict__ X, const float *__restrict__ U,
+                                                    const float *__restrict__ NW, int K, float eps, uint32_t *zero,
+                                                    int n_zero)
+{
+    __shared__ float red[16];
+    const int n4 = K >> 2;
+    const int64_t r4 = (int64_t)blockIdx.x * n4;
+    // every load of the row issued first, through buffer resources over the
+    // row (and the norm weights): a float4 past K reads zeros, so no load
+    // waits behind a branch or behind another's arithmetic
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)((const float4 *)X + r4), (short)0, K * 4, kRawBufWord3);
+    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(MODE == XS_SWIGLU ? (const float4 *)U + r4 : (const float4 *)X + r4), (short)0, K * 4, kRawBufWord3);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(MODE == XS_NORM ? NW : X), (short)0, K * 4, kRawBufWord3);
+    float4 v[NV], wv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int o = (int)(threadIdx.x + NT * j) * 16;
+        v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
+        if constexpr (MODE == XS_SWIGLU)
+            wv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
+        if constexpr (MODE == XS_NORM)
+            wv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        if constexpr (MODE == XS_SWIGLU) {
+            const float4 u = wv[j];
+            v[j].x = (v[j].x / (1.0f + expf(-v[j].x))) * u.x;
+            v[j].y = (v[j].y / (1.0f + expf(-v[j].y))) * u.y;
+            v[j].z = (v[j].z / (1.0f + expf(-v[j].z))) * u.z;
+            v[j].w = (v[j].w / (1.0f + expf(-v[j].w))) * u.w;
+        }
+        if constexpr (MODE == XS_NORM)
+            ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    }
+    float scale = 1.f;
+    if constexpr (MODE == XS_NORM) {
+        ss = block_reduce<false>(ss, red);
+        scale = 1.0f / sqrtf(ss / (float)K + eps);
+    }
+    float am = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        if constexpr (MODE == XS_NORM) {
+            const float4 w4 = wv[j];
+            v[j] = make_float4(v[j].x * scale * w4.x, v[j].y * scale * w4.y, v[j].z * scale * w4.z,
+                               v[j].w * scale * w4.w);
+        }
+        am = fmaxf(am, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
+    }
+    am = block_reduce<true>(am, red);
+    // 2^e with a * 2^e in [2^14, 2^15); e = 0 for a zero or non-finite row
+    int e = 0;
+    if (am > 0.f && am <= 3.4028235e38f) {
+        int ea;
+        (void)frexpf(am, &ea);  // am = f * 2^ea, f in [0.5, 1)
+        e = 15 - ea;
+    }
+    if (threadIdx.x == 0) Rs[blockIdx.x] = ldexpf(1.0f, -e);
+    if (OPS && blockIdx.x == 0)
+        for (int j = threadIdx.x; j < n_zero; j += NT) zero[j] = 0;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + NT * j;
+        if (NT * j >= n4) break;  // uniform: no lane of this or a later j is live
+        const float y[4] = {ldexpf(v[j].x, e), ldexpf(v[j].y, e), ldexpf(v[j].z, e), ldexpf(v[j].w, e)};
+        _Float16 h[4], l[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            h[q] = (_Float16)y[q];
+            l[q] = (_Float16)(y[q] - (float)h[q]);
+            if (OPS && fabsf(y[q]) > 65504.0f) l[q] = (_Float16)0.0f;
+        }
+        // the block's sum over its 8 lanes (octets are wholly live or dead)
+        float s = (y[0] + y[1]) + (y[2] + y[3]);
+        s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xB1, 0xF, 0xF, false));  // [1,0,3,2]
+        s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4E, 0xF, 0xF, false));  // [2,3,0,1]
+        s += __shfl_xor(s, 4, 64);
+        if constexpr (OPS) {
+            // float4 i is block i / 8, weights 4 (i % 8) .. of it: operand lane
+            // row + 16 (i % 4), half (i % 8) / 4 of its 16 bytes, order 0, 2, 1, 3
+            if (i < n4) {
+                const int64_t b = (int64_t)(blockIdx.x >> 4) * (n4 >> 3) + (i >> 3);
+                const int m = blockIdx.x & 15;
+                const int64_t o = ((b * 128 + m + 16 * (i & 3)) << 1) + ((i >> 2) & 1);
+                Ah[o] = make_uint2(__builtin_bit_cast(uint32_t, h2{h[0], h[2]}), __builtin_bit_cast(uint32_t, h2{h[1], h[3]}));
+                Ah[o + 128] = make_uint2(__builtin_bit_cast(uint32_t, h2{l[0], l[2]}), __builtin_bit_cast(uint32_t, h2{l[1], l[3]}));
+                if (Sx && (i & 7) == 0) Sx[b * 16 + m] = s;
+            }
+        } else if (i < n4) {
+            Ah[r4 + i] = make_uint2(__builtin_bit_cast(uint32_t, h2{h[0], h[1]}), __builtin_bit_cast(uint32_t, h2{h[2], h[3]}));
+            Al[r4 + i] = make_uint2(__builtin_bit_cast(uint32_t, h2{l[0], l[1]}), __builtin_bit_cast(uint32_t, h2{l[2], l[3]}));
+            if (Sx && (i & 7) == 0) Sx[r4 / 8 + (i >> 3)] = s;
+        }
+    }
+}
+
+}  // namespace
+
+}  // namespace holo

@@ -48,8 +48,23 @@ bool exact_init();
 void exact_release();
 // With NW, the rows of X are RMS-normed first (weight NW, K <= 16384, 16-byte
 // aligned), as holo_rms_norm_rows computes them, inside the activation halves.
-void exact_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
+// false, with nothing launched, only for under 64 rows that few_rows.hip
+// does not take (no scratch, or a matrix too large).
+bool exact_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
                    const float *U, const float *R, int M, int K, const float *NW = nullptr, float eps = 0.f);
+// What the exact product's 64 x 256 tiles take, in us (an estimate), and
+// whether they fill the chip.
+float exact_tiles_us(int type, int N, int M, int nb, bool *full);
+// The same for a few rows (few_rows.hip): whether a row count goes there
+// instead of to one GEMV per row, the product (false: nothing launched), and
+// the release of its scratch (all of it; a stream's, before it is destroyed).
+bool few_rows_take(int M);
+bool few_rows_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
+                      const float *U, const float *R, int M, int K, const float *NW, float eps);
+void few_rows_release();
+void few_rows_drop_stream(hipStream_t st);
+// The GEMVs run their default activation mode (holo_gemv_set_xmode).
+bool gemv_default_mode();
 // The exact route for nmat matrices of rows RMS-normed on the way in, when
 // the prefill mode and the shapes take it; false (nothing launched) otherwise.
 bool exact_product_normed(float *const *Y, const void *const *W, const int *types, const int *N, int nmat,

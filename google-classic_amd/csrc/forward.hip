@@ -45,12 +45,11 @@ void norm_or_copy(float *dst, const float *x, const float *w, int rows, int n, f
 
 bool fused_gemv_type(int t) { return t == HOLO_TYPE_Q4_0 || t == HOLO_TYPE_Q8_0 || t == HOLO_TYPE_Q4_K; }
 
-// The batched product takes the rows: at least 64, not in exact mode, in_dim
-// whole blocks of the type (holo_matmul_batch: Q4_0 on its own kernels, the
-// other types on a dequantised f16 panel).
+// The batched product takes the rows (holo_matmul_batch): not in exact mode,
+// in_dim whole blocks of the type; under 64 rows what few_rows.hip takes.
 bool gemm_rows(int type, int rows, int in_dim, int exact)
 {
-    if (rows < 64 || exact) return false;
+    if (exact || (rows < 64 && (!few_rows_take(rows) || type == HOLO_TYPE_F32 || in_dim > 16384))) return false;
     switch (type) {
     case HOLO_TYPE_Q4_0:
     case HOLO_TYPE_Q8_0:
@@ -145,7 +144,7 @@ void holo_matmul_rows(float *Y, const void *W, const float *X, int rows, int out
                       int exact)
 {
     if (rows <= 0 || out_dim <= 0) return;
-    if (gemm_rows(type, rows, in_dim, exact)) {
+    if (gemm_rows(type, rows, in_dim, exact) && (rows >= 64 || (W && X && Y))) {
         holo_matmul_batch(Y, W, X, rows, out_dim, in_dim, type);
         return;
     }

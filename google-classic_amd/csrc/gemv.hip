@@ -811,6 +811,8 @@ static const Tuning &tuning()
     return g_tune;
 }
 
+bool gemv_default_mode() { return tuning().xmode == XM_MFMA; }
+
 constexpr int kMaxLdsBytes = 64 * 1024;
 constexpr size_t kMaxMfmaLds = 160 * 1024;  // MI355X: 160 KB of LDS per workgroup
 

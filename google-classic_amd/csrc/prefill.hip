@@ -855,6 +855,10 @@ static bool exact_fits(const void *const *W, const int *types, int nmat, const f
 
 static bool exact_mode() { return g_prefill_mode == HOLO_PREFILL_EXACT; }
 
+// M rows go to the exact product: under 64 in every mode (the modes choose
+// among the products of 64 rows and more).
+static bool exact_rows(int M) { return M < 64 ? few_rows_take(M) : exact_mode(); }
+
 extern "C" {
 
 void holo_prefill_set_q8_kernel(int kind)
@@ -875,13 +879,12 @@ namespace holo {
 bool exact_product_normed(float *const *Y, const void *const *W, const int *types, const int *N, int nmat,
                           const float *X, const float *NW, float eps, int M, int K)
 {
-    if (M < 64 || !exact_mode() || !Y || !W || !types || !N || !NW || ((uintptr_t)NW & 15u) || K > 1024 * 16 ||
+    if (!exact_rows(M) || !Y || !W || !types || !N || !NW || ((uintptr_t)NW & 15u) || K > 1024 * 16 ||
         !multi_fits(N, nmat) || !exact_fits(W, types, nmat, X, nullptr, M, K))
         return false;
     for (int i = 0; i < nmat; i++)
         if (!Y[i]) return false;
-    exact_product(Y, W, types, N, nmat, X, nullptr, nullptr, M, K, NW, eps);
-    return true;
+    return exact_product(Y, W, types, N, nmat, X, nullptr, nullptr, M, K, NW, eps);
 }
 
 }  // namespace holo
@@ -894,10 +897,9 @@ void holo_matmul_batch_q4_0(float *Y, const void *W, const float *X, int M, int 
 {
     if (M <= 0 || N <= 0) return;
     const int t = HOLO_TYPE_Q4_0;
-    if (M >= 64 && exact_mode() && exact_fits(&W, &t, 1, X, nullptr, M, K)) {
-        exact_product(&Y, &W, &t, &N, 1, X, nullptr, nullptr, M, K);
+    if (exact_rows(M) && exact_fits(&W, &t, 1, X, nullptr, M, K) &&
+        exact_product(&Y, &W, &t, &N, 1, X, nullptr, nullptr, M, K))
         return;
-    }
     if (M < 64 || exact_mode()) {
         for (int m = 0; m < M; m++) cuda_matmul_q4_0(Y + (int64_t)m * N, W, X + (int64_t)m * K, N, K);
         return;
@@ -922,10 +924,9 @@ void holo_matmul_batch_q4_0_add(float *Y, const void *W, const float *X, const f
         return;
     }
     const int t = HOLO_TYPE_Q4_0;
-    if (M >= 64 && exact_mode() && exact_fits(&W, &t, 1, X, nullptr, M, K)) {
-        exact_product(&Y, &W, &t, &N, 1, X, nullptr, R, M, K);
+    if (exact_rows(M) && exact_fits(&W, &t, 1, X, nullptr, M, K) &&
+        exact_product(&Y, &W, &t, &N, 1, X, nullptr, R, M, K))
         return;
-    }
     if (M < 64 || exact_mode()) {
         for (int m = 0; m < M; m++)
             holo_matmul_add(Y + (int64_t)m * N, W, X + (int64_t)m * K, R + (int64_t)m * N, N, K, HOLO_TYPE_Q4_0);
@@ -952,10 +953,9 @@ void holo_matmul_batch_q4_0_swiglu_add(float *Y, const void *W, float *G, const 
         return;
     }
     const int t = HOLO_TYPE_Q4_0;
-    if (M >= 64 && exact_mode() && exact_fits(&W, &t, 1, G, U, M, K)) {
-        exact_product(&Y, &W, &t, &N, 1, G, U, R, M, K);
+    if (exact_rows(M) && exact_fits(&W, &t, 1, G, U, M, K) &&
+        exact_product(&Y, &W, &t, &N, 1, G, U, R, M, K))
         return;
-    }
     if (M >= 64 && g_prefill_mode == HOLO_PREFILL_F16 && !(((uintptr_t)G | (uintptr_t)U) & 15u)) {
         gemm_multi(&Y, &W, &N, 1, nullptr, G, M, K, U, R);
         return;
@@ -973,10 +973,9 @@ void holo_matmul_batch_q4_0_multi(float *const *Y, const void *const *W, const i
         return;
     }
     const int T[3] = {HOLO_TYPE_Q4_0, HOLO_TYPE_Q4_0, HOLO_TYPE_Q4_0};
-    if (M >= 64 && exact_mode() && exact_fits(W, T, nmat, X, nullptr, M, K)) {
-        exact_product(Y, W, T, N, nmat, X, nullptr, nullptr, M, K);
+    if (exact_rows(M) && exact_fits(W, T, nmat, X, nullptr, M, K) &&
+        exact_product(Y, W, T, N, nmat, X, nullptr, nullptr, M, K))
         return;
-    }
     if (M < 64 || exact_mode()) {
         for (int i = 0; i < nmat; i++) holo_matmul_batch_q4_0(Y[i], W[i], X, M, N[i], K, scratch_q8);
         return;
@@ -1071,10 +1070,9 @@ void holo_matmul_batch(float *Y, const void *W, const float *X, int M, int N, in
         HOLO_REJECT("holo_matmul_batch: null pointer");
         return;
     }
-    if (M >= 64 && exact_mode() && exact_fits(&W, &type, 1, X, nullptr, M, K)) {
-        exact_product(&Y, &W, &type, &N, 1, X, nullptr, nullptr, M, K);
+    if (exact_rows(M) && exact_fits(&W, &type, 1, X, nullptr, M, K) &&
+        exact_product(&Y, &W, &type, &N, 1, X, nullptr, nullptr, M, K))
         return;
-    }
     if (M < 64 || exact_mode() || !panel_ok(type, K) || !panel_src_aligned(W, type) || ((uintptr_t)X & 15u)) {
         for (int m = 0; m < M; m++) holo_matmul(Y + (int64_t)m * N, W, X + (int64_t)m * K, N, K, type);
         return;
@@ -1095,10 +1093,9 @@ void holo_matmul_batch_multi(float *const *Y, const void *const *W, const int *N
         return;
     }
     const int T[3] = {type, type, type};
-    if (M >= 64 && exact_mode() && exact_fits(W, T, nmat, X, nullptr, M, K)) {
-        exact_product(Y, W, T, N, nmat, X, nullptr, nullptr, M, K);
+    if (exact_rows(M) && exact_fits(W, T, nmat, X, nullptr, M, K) &&
+        exact_product(Y, W, T, N, nmat, X, nullptr, nullptr, M, K))
         return;
-    }
     bool ok = M >= 64 && !exact_mode() && panel_ok(type, K) && !((uintptr_t)X & 15u);
     for (int i = 0; i < nmat; i++) ok = ok && Y[i] && W[i] && panel_src_aligned(W[i], type);
     if (!ok) {
@@ -1122,10 +1119,9 @@ void holo_matmul_batch_multi_types(float *const *Y, const void *const *W, const 
         holo_matmul_batch_multi(Y, W, N, nmat, X, M, K, types[0]);
         return;
     }
-    if (M >= 64 && exact_mode() && exact_fits(W, types, nmat, X, nullptr, M, K)) {
-        exact_product(Y, W, types, N, nmat, X, nullptr, nullptr, M, K);
+    if (exact_rows(M) && exact_fits(W, types, nmat, X, nullptr, M, K) &&
+        exact_product(Y, W, types, N, nmat, X, nullptr, nullptr, M, K))
         return;
-    }
     bool ok = M >= 64 && !exact_mode() && !((uintptr_t)X & 15u);
     for (int i = 0; i < nmat; i++)
         ok = ok && Y[i] && W[i] && panel_ok(types[i], K) && panel_src_aligned(W[i], types[i]);
@@ -1147,10 +1143,9 @@ void holo_matmul_batch_add(float *Y, const void *W, const float *X, const float 
         HOLO_REJECT("holo_matmul_batch_add: null pointer");
         return;
     }
-    if (M >= 64 && exact_mode() && exact_fits(&W, &type, 1, X, nullptr, M, K)) {
-        exact_product(&Y, &W, &type, &N, 1, X, nullptr, R, M, K);  // the add in the GEMM's store
-        return;
-    }
+    if (exact_rows(M) && exact_fits(&W, &type, 1, X, nullptr, M, K) &&
+        exact_product(&Y, &W, &type, &N, 1, X, nullptr, R, M, K))
+        return;  // the add in the GEMM's store
     if (M >= 64 && !exact_mode() && panel_ok(type, K) && panel_src_aligned(W, type) && !((uintptr_t)X & 15u)) {
         gemm_panel(&Y, &W, &N, 1, X, M, K, type, nullptr, R);  // the add in the GEMM's store
         return;
@@ -1178,10 +1173,9 @@ void holo_matmul_batch_swiglu_add(float *Y, const void *W, float *G, const float
         HOLO_REJECT("holo_matmul_batch_swiglu_add: null pointer");
         return;
     }
-    if (M >= 64 && exact_mode() && exact_fits(&W, &type, 1, G, U, M, K)) {
-        exact_product(&Y, &W, &type, &N, 1, G, U, R, M, K);  // silu(G) * U in the activation halves
-        return;
-    }
+    if (exact_rows(M) && exact_fits(&W, &type, 1, G, U, M, K) &&
+        exact_product(&Y, &W, &type, &N, 1, G, U, R, M, K))
+        return;  // silu(G) * U in the activation halves
     if (M >= 64 && !exact_mode() && panel_ok(type, K) && panel_src_aligned(W, type) &&
         !(((uintptr_t)G | (uintptr_t)U) & 15u)) {
         gemm_panel(&Y, &W, &N, 1, G, M, K, type, U, R);  // silu(G) * U in the activation panel

@@ -31,7 +31,8 @@
 // stage's global loads in registers while the current one is multiplied.
 #include "common.h"
 #include "quant_blocks.h"
-#include "block_reduce.h"
+#include "activation_split.h"
+#include "exact_blocks.h"
 
 #include <hip/hip_ext.h>
 #include <algorithm>
@@ -46,17 +47,6 @@
 namespace holo {
 
 namespace {
-
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef uint32_t v3u __attribute__((ext_vector_type(3)));
-
-// Weight source of one launch (EW_Q6R: Q6_K repacked for the second tiling).
-enum ExactW { EW_Q4_0 = 0, EW_Q8_0 = 1, EW_Q4_K = 2, EW_P16 = 3, EW_F16 = 4, EW_Q6_K = 5, EW_Q6R = 6 };
-
-constexpr int kExactMats = 3;
 
 struct ExactArgs {
     float *Y[kExactMats];
@@ -78,36 +68,6 @@ struct ExactMat {
     int nbase, N;
     int64_t w_bytes;
 };
-
-// ---- integers of a block in f16 ----------------------------------------------------
-// v_perm pairs a byte with 0x64, giving the f16 value 1024 + byte; one
-// packed f16 add removes the bias, exactly.
-
-__device__ __forceinline__ uint32_t f16_pair(uint32_t bytes, uint32_t sel, _Float16 bias)
-{
-    const h2 b2 = {bias, bias};
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, bytes, sel)) + b2);
-}
-
-// Eight nibbles of x (four bytes): lo[0..1] = low nibbles (k = 4j..4j+3 of the
-// block), hi[0..1] = high nibbles (k = 16+4j..), each as f16 (nibble + off).
-__device__ __forceinline__ void nibbles_f16(uint32_t x, _Float16 off, uint32_t lo[2], uint32_t hi[2])
-{
-    const uint32_t t0 = x & 0x0F0F0F0Fu, t1 = (x >> 4) & 0x0F0F0F0Fu;
-    const _Float16 bias = (_Float16)(-1024.0f) + off;
-    lo[0] = f16_pair(t0, 0x04010400u, bias);
-    lo[1] = f16_pair(t0, 0x04030402u, bias);
-    hi[0] = f16_pair(t1, 0x04010400u, bias);
-    hi[1] = f16_pair(t1, 0x04030402u, bias);
-}
-
-// Four signed bytes as f16: byte ^ 0x80 is q + 128 in 0..255.
-__device__ __forceinline__ void int8s_f16(uint32_t x, uint32_t out[2])
-{
-    const uint32_t t = x ^ 0x80808080u;
-    out[0] = f16_pair(t, 0x04010400u, (_Float16)-1152.0f);
-    out[1] = f16_pair(t, 0x04030402u, (_Float16)-1152.0f);
-}
 
 template <int WM, int WN, int S>
 struct XGeo {
@@ -589,110 +549,6 @@ __global__ __launch_bounds__(256, OCC) void gemm_exact_k(ExactArgs a)
                 }
             }
         }
-}
-
-// ---- the activation halves: Ah, Al [M][K] f16, block sums Sx [M][K/32], row scales Rs [M] ----
-// One workgroup per row.  The row's values y (x; silu(g) * u as
-// cuda_silu_mul computes it, cuda_ops.cu:304-314; or the RMS-normed row,
-// rms_norm_rows4_k's arithmetic: thread t sums the squares of float4s
-// t + 256 j, the same workgroup reduction, x * scale * w, so the normed
-// values are the bits the separate norm writes) are scaled by a power of two
-// 2^e chosen from the row's largest magnitude a: a * 2^e lies in
-// [2^14, 2^15).  The halves then never overflow f16 (|y| up to fp32's range
-// is taken) and the low half is a normal f16 for every value above
-// a * 2^-17, so x - xh - xl stays within 2^-22 |x| there and within
-// a * 2^-40 below.  The product's store multiplies by Rs = 2^-e (exact).  A
-// 32-block is the 8 float4 of 8 adjacent lanes (K % 32 == 0); Sx holds the
-// block sums of the scaled values (for the Q4_K min term).
-enum XSplitMode { XS_PLAIN = 0, XS_SWIGLU = 1, XS_NORM = 2 };
-
-template <int NV, int MODE, int NT = 256>
-__global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2 *__restrict__ Al,
-                                                    float *__restrict__ Sx, float *__restrict__ Rs,
-                                                    const float *__restrict__ X, const float *__restrict__ U,
-                                                    const float *__restrict__ NW, int K, float eps)
-{
-    __shared__ float red[16];
-    const int n4 = K >> 2;
-    const int64_t r4 = (int64_t)blockIdx.x * n4;
-    // every load of the row issued first, through buffer resources over the
-    // row (and the norm weights): a float4 past K reads zeros, so no load
-    // waits behind a branch or behind another's arithmetic
-    const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc((void *)((const float4 *)X + r4), (short)0, K * 4, kXBufWord3);
-    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(MODE == XS_SWIGLU ? (const float4 *)U + r4 : (const float4 *)X + r4), (short)0, K * 4, kXBufWord3);
-    const __amdgpu_buffer_rsrc_t rw =
-        __builtin_amdgcn_make_buffer_rsrc((void *)(MODE == XS_NORM ? NW : X), (short)0, K * 4, kXBufWord3);
-    float4 v[NV], wv[NV];
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int o = (int)(threadIdx.x + NT * j) * 16;
-        v[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
-        if constexpr (MODE == XS_SWIGLU)
-            wv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
-        if constexpr (MODE == XS_NORM)
-            wv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
-    }
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        if constexpr (MODE == XS_SWIGLU) {
-            const float4 u = wv[j];
-            v[j].x = (v[j].x / (1.0f + expf(-v[j].x))) * u.x;
-            v[j].y = (v[j].y / (1.0f + expf(-v[j].y))) * u.y;
-            v[j].z = (v[j].z / (1.0f + expf(-v[j].z))) * u.z;
-            v[j].w = (v[j].w / (1.0f + expf(-v[j].w))) * u.w;
-        }
-        if constexpr (MODE == XS_NORM)
-            ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
-    }
-    float scale = 1.f;
-    if constexpr (MODE == XS_NORM) {
-        ss = block_reduce<false>(ss, red);
-        scale = 1.0f / sqrtf(ss / (float)K + eps);
-    }
-    float am = 0.f;
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        if constexpr (MODE == XS_NORM) {
-            const float4 w4 = wv[j];
-            v[j] = make_float4(v[j].x * scale * w4.x, v[j].y * scale * w4.y, v[j].z * scale * w4.z,
-                               v[j].w * scale * w4.w);
-        }
-        am = fmaxf(am, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
-    }
-    am = block_reduce<true>(am, red);
-    // 2^e with a * 2^e in [2^14, 2^15); e = 0 for a zero or non-finite row
-    int e = 0;
-    if (am > 0.f && am <= 3.4028235e38f) {
-        int ea;
-        (void)frexpf(am, &ea);  // am = f * 2^ea, f in [0.5, 1)
-        e = 15 - ea;
-    }
-    if (threadIdx.x == 0) Rs[blockIdx.x] = ldexpf(1.0f, -e);
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int i = threadIdx.x + NT * j;
-        if (NT * j >= n4) break;  // uniform: no lane of this or a later j is live
-        const float y[4] = {ldexpf(v[j].x, e), ldexpf(v[j].y, e), ldexpf(v[j].z, e), ldexpf(v[j].w, e)};
-        _Float16 h[4], l[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            h[q] = (_Float16)y[q];
-            l[q] = (_Float16)(y[q] - (float)h[q]);
-        }
-        // the block's sum over its 8 lanes (octets are wholly live or dead)
-        float s = (y[0] + y[1]) + (y[2] + y[3]);
-        s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0xB1, 0xF, 0xF, false));  // [1,0,3,2]
-        s += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x4E, 0xF, 0xF, false));  // [2,3,0,1]
-        s += __shfl_xor(s, 4, 64);
-        if (i < n4) {
-            Ah[r4 + i] = make_uint2(__builtin_bit_cast(uint32_t, h2{h[0], h[1]}), __builtin_bit_cast(uint32_t, h2{h[2], h[3]}));
-            Al[r4 + i] = make_uint2(__builtin_bit_cast(uint32_t, h2{l[0], l[1]}), __builtin_bit_cast(uint32_t, h2{l[2], l[3]}));
-            if (Sx && (i & 7) == 0) Sx[r4 / 8 + (i >> 3)] = s;
-        }
-    }
 }
 
 // ---- Q6_K integer panel: (q - 32) in f16 [N][K] and the group scales d*sc [N][K/16] ----
@@ -1497,6 +1353,15 @@ void launch_exact_for(const ExactArgs &a)
 
 uint32_t *g_x2_cnt = nullptr;  // tile counters of the split form, zero between launches
 
+// Ranges per row of tiles.
+static int x2_ranges(int nct, int nst, int ntm)
+{
+    const int64_t U = (int64_t)nct * nst;
+    int64_t gr = std::max(1, 2 * num_cus() / ntm);
+    gr = std::min(gr, U / kX2MinStages);
+    return (int)std::max<int64_t>(1, std::min(gr, (int64_t)kX2MaxSplit * nct));
+}
+
 // The second tiling: about 2 workgroups per CU (both resident), the same
 // number per row of tiles, share the stages evenly, with ranges of at least
 // kX2MinStages stages and at most about kX2MaxSplit workgroups per tile; a
@@ -1511,9 +1376,7 @@ void launch_exact2(X2Args a)
     a.nst = (a.nb + S - 1) / S;
     const int nct = a.tiles / a.ntm;
     const int64_t U = (int64_t)nct * a.nst;  // items of a row of tiles
-    int64_t gr = std::max(1, 2 * num_cus() / a.ntm);
-    gr = std::min(gr, U / kX2MinStages);
-    gr = std::max<int64_t>(1, std::min(gr, (int64_t)kX2MaxSplit * nct));
+    int64_t gr = x2_ranges(nct, a.nst, a.ntm);
     if (!g_x2_cnt || a.tiles > kX2Counters) gr = nct;  // whole tiles only
     a.gr = (int)gr;
     const int64_t NG = (int64_t)a.ntm * gr;
@@ -1570,6 +1433,21 @@ int exact_kind(int type)
 
 }  // namespace
 
+// About what the second tiling takes, us: 20 and a time per
+// stage of the longest range, more where ranges share a CU (Q4_0, measured:
+// 100 x 4096 x 4096 in 41, 192 x 11008 x 4096 in 73, 128 x 4096 x 11008 in 74;
+// 100 x 4096 x 14336 Q4_K in 104, 128 x 4096 x 11008 Q6_K in 107).
+// `full`: the launch puts both of its workgroups on every CU (above 256 rows,
+// one: 958 x 1427 x 10240 Q8_0 then takes 117, the few-row tiles 140).
+float exact_tiles_us(int type, int N, int M, int nb, bool *full)
+{
+    const int ntm = (M + 63) / 64, nct = (N + 255) / 256, nst = (nb + 1) / 2;
+    const int gr = x2_ranges(nct, nst, ntm);
+    *full = M > 256 ? ntm * gr > num_cus() : ntm * gr >= 2 * num_cus();
+    const float stage = type == HOLO_TYPE_Q4_K ? 1.5f : type == HOLO_TYPE_Q6_K ? 2.0f : type == HOLO_TYPE_Q8_0 ? 1.7f : 1.25f;
+    return 20.f + stage * (float)((int64_t)nct * nst) / (float)gr * std::max(1.f, (float)(ntm * gr) / (float)num_cus());
+}
+
 bool exact_init()
 {
     if (g_x2_cnt) return true;
@@ -1620,6 +1498,7 @@ void q6r_repack(void *out, const void *W, int N, int K)
 
 void exact_release()
 {
+    few_rows_release();
     if (g_x2_cnt) (void)hipFree(g_x2_cnt);
     g_x2_cnt = nullptr;
     prepared_release_all();
@@ -1647,9 +1526,13 @@ bool exact_ok(int type, int K, const void *W)
 // nmat matrices sharing the activations; every type must pass exact_ok, and
 // with several matrices of one type every N[i] must be a multiple of 128.
 // Matrices of one type share a launch; the activation halves are built once.
-void exact_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
+// Few rows run few_rows.hip's kernels; false (nothing launched) when under
+// 64 rows those do not take the call.
+bool exact_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
                    const float *U, const float *R, int M, int K, const float *NW, float eps)
 {
+    if (!exact_v1() && few_rows_product(Y, W, types, N, nmat, X, U, R, M, K, NW, eps)) return true;
+    if (M < 64) return false;
     const int nb = K / 32;
     const size_t half = ((size_t)M * K * 2 + 255) & ~(size_t)255;
     const size_t sxb = ((size_t)M * nb * 4 + 255) & ~(size_t)255;
@@ -1657,7 +1540,7 @@ void exact_product(float *const *Y, const void *const *W, const int *types, cons
     void *aws = workspace(1, abytes);
     const bool own_a = aws == nullptr;
     if (own_a) HOLO_CHECK(hipMallocAsync(&aws, abytes, stream()));
-    if (!aws) return;
+    if (!aws) return true;
     _Float16 *Ah = (_Float16 *)aws, *Al = (_Float16 *)((uint8_t *)aws + half);
     float *Sx = (float *)((uint8_t *)aws + 2 * half);
     float *Rs = (float *)((uint8_t *)aws + 2 * half + sxb);
@@ -1682,7 +1565,7 @@ void exact_product(float *const *Y, const void *const *W, const int *types, cons
     // one workgroup per row, K <= 16384 (exact_ok): the row in registers
     auto split = [&](auto kern, int nt) {
         hipLaunchKernelGGL(kern, dim3(M), dim3(nt), 0, stream(), (uint2 *)Ah, (uint2 *)Al, need_sx ? Sx : nullptr,
-                           Rs, X, U, NW, K, eps);
+                           Rs, X, U, NW, K, eps, nullptr, 0);
     };
     // the normed form keeps rms_norm_rows4_k's 256 threads (its sum of squares
     // in the same order); the others reduce only a maximum, so their threads
@@ -1701,7 +1584,7 @@ void exact_product(float *const *Y, const void *const *W, const int *types, cons
         pws = workspace(0, pbytes);
         own_p = pws == nullptr;
         if (own_p) HOLO_CHECK(hipMallocAsync(&pws, pbytes, stream()));
-        if (!pws) return;
+        if (!pws) return true;
         size_t off = 0;
         for (int i = 0; i < nmat; i++) {
             if (kinds[i] == EW_Q6R) {
@@ -1813,6 +1696,7 @@ void exact_product(float *const *Y, const void *const *W, const int *types, cons
     }
     if (own_p) HOLO_CHECK(hipFreeAsync(pws, stream()));
     if (own_a) HOLO_CHECK(hipFreeAsync(aws, stream()));
+    return true;
 }
 
 }  // namespace holo

@@ -248,7 +248,9 @@ void *holo_stream_create(void)
 
 void holo_stream_destroy(void *s)
 {
-    if (s) HOLO_CHECK(hipStreamDestroy((hipStream_t)s));
+    if (!s) return;
+    holo::few_rows_drop_stream((hipStream_t)s);
+    HOLO_CHECK(hipStreamDestroy((hipStream_t)s));
 }
 
 void *holo_event_create(void)

@@ -223,19 +223,23 @@ int holo_gemm_q4_0_q8_0_noalloc(float *Y, const void *W, const void *Xq, int M, 
 #define HOLO_Q8_KERNEL_I8 1
 void holo_prefill_set_q8_kernel(int kind);
 int holo_prefill_get_q8_kernel(void);
-/* Y[M][N] = X[M][K] . W[N][K]^T for W in Q4_0.  M >= 64 runs, by the mode
- * set below: the exact product (HOLO_PREFILL_EXACT, the default: each row of
+/* Y[M][N] = X[M][K] . W[N][K]^T for W in Q4_0.  3 <= M < 64 runs the exact
+ * product below in tiles for few rows (in the default GEMV activation mode, K
+ * <= 16384 and a multiple of 32, X 16-byte aligned; a scratch buffer per
+ * stream that the library keeps, stream-ordered under capture; without memory
+ * for it M GEMVs).  M >= 64 runs, by the mode set below: the exact product (HOLO_PREFILL_EXACT, the default: each row of
  * X scaled by a power of two and split into two f16 halves, x - xh - xl
  * within 2^-22 |x|, times the block's integers, exact in f16, on the f16
  * matrix cores, block scales applied in fp32 in block order; fp32 accuracy,
  * within 1e-3 of the CPU path; X 16-byte aligned and K <= 16384, else M
- * GEMVs; the K blocks of each row of tiles are dealt evenly to about two
+ * GEMVs; the tiles for few rows where they are the faster ones, else the
+ * K blocks of each row of tiles are dealt evenly to about two
  * workgroups per CU, and a tile whose blocks two or more workgroups share
  * is the sum of their parts in K order, so the result depends on the
  * launch's shape and the CU count but not on timing), the f16 product below
  * (HOLO_PREFILL_F16) or the Q8_0
- * product above (HOLO_PREFILL_Q8_0: X quantised to Q8_0).  M < 64 runs M
- * GEMVs.                                                                     */
+ * product above (HOLO_PREFILL_Q8_0: X quantised to Q8_0).  Other calls with
+ * M < 64 run M GEMVs.                                                        */
 void holo_matmul_batch_q4_0(float *Y, const void *W, const float *X, int M, int N, int K,
                             void *scratch_q8);
 /* The same over nmat = 1..3 Q4_0 matrices that multiply the same X in one
@@ -265,8 +269,9 @@ void holo_gemm_q4_0_f16_multi(float *const *Y, const void *const *W, const int *
  * analogue of holo_matmul_add): Y = R + X . W^T, and Y = R + (silu(G) * U) .
  * W^T with silu(g) * u as cuda_silu_mul computes it -- the add in the
  * GEMM's output store, the SwiGLU in its f16 activation panel.  Y may alias
- * R.  M < 64 runs GEMVs; outside the f16 product (Q8_0 mode, misaligned G/U,
- * M < 64) the SwiGLU is stored into G first, so G's contents are not kept. */
+ * R.  M < 64 as above; outside the exact and f16 products (Q8_0 mode,
+ * misaligned G/U, GEMVs) the SwiGLU is stored into G first, so G's contents
+ * are not kept.                                                            */
 void holo_matmul_batch_q4_0_add(float *Y, const void *W, const float *X, const float *R, int M, int N, int K);
 void holo_matmul_batch_q4_0_swiglu_add(float *Y, const void *W, float *G, const float *U, const float *R,
                                        int M, int N, int K);
@@ -279,18 +284,18 @@ void holo_matmul_batch_q4_0_multi(float *const *Y, const void *const *W, const i
                                   const float *X, int M, int K, void *scratch_q8);
 /* The batched products for any weight type the GEMVs serve (Q4_0, Q8_0, Q4_K,
  * Q6_K, F16, F32), with the contracts of the Q4_0 calls above.  Q4_0 goes to
- * them.  Every other type, for M >= 64 and K whole blocks (Q4_K, Q6_K: K a
+ * them.  Every other type, for M >= 3 and K whole blocks (Q4_K, Q6_K: K a
  * multiple of 256) up to 16384, runs the exact product by default (the block
- * integers against the two f16 halves of X, block scales in fp32); in
- * HOLO_PREFILL_F16 mode it is dequantised into an f16 panel
+ * integers against the two f16 halves of X, block scales in fp32; F32
+ * matrices run GEMVs); in HOLO_PREFILL_F16 mode, for M >= 64, it is dequantised into an f16 panel
  * (holo_dequant_f16, N*K*2 bytes per matrix) and multiplied on the f16
  * product.  Workspaces live in device buffers the library keeps and grows
  * (hipMalloc, outside graph capture; under capture a stream-ordered
  * allocation per call); calls on one stream reuse them in order.  Otherwise
  * one holo_matmul GEMV per row.  The multi forms take up to 3 matrices
  * sharing X (with several, every N a multiple of 128); an output equals the
- * single call's bit for bit when neither launch shares a tile's K blocks
- * between workgroups (for Q4_0, Q8_0, Q4_K, Q6_K and F16 that is when the K
+ * single call's bit for bit when both run the same tiles (few rows or not)
+ * and neither launch shares a tile's K blocks between workgroups (for Q4_0, Q8_0, Q4_K, Q6_K and F16 that is when the K
  * blocks per row of tiles split evenly into whole tiles per workgroup; Q6_K
  * matrices are first repacked into the workspace), else it is
  * within the product's error bound.  No reference counterpart (the
@@ -318,7 +323,8 @@ void holo_matmul_batch_swiglu_add(float *Y, const void *W, float *G, const float
  * in its workspace first.  holo_prefill_prepare allocates that copy of W
  * [N][K] (N*K bytes, hipMalloc), writes it, waits for it, and keeps it until
  * holo_prefill_release(W): every later exact batched product on W with the
- * same N and K reads the copy, with the same bits as the per-call form.  W
+ * same N and K that would repack it (few-row tiles read W as it is) reads the
+ * copy, with the same bits as the per-call form.  W
  * must not change and must not be freed while registered, and a graph
  * captured while W was registered reads the copy: destroy such graphs
  * before releasing W.  Returns 0 (also

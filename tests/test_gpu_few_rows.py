@@ -1,0 +1,182 @@
+"""GPU parity of the exact product for a few rows (few_rows.hip), through
+holo_matmul_batch and its forms.
+
+Truth and elementwise bar are those of test_gpu_batch_exact: the float64
+product of the fp32 activations and the bit-exact dequantised weights, within
+(K/32 + 70) 2^-24 sum_k |x w| (doubled for Q4_K).  The waves' eight partial
+sums, up to 32 over four parts of K, replace as many roundings of the
+block-order sum, so the bar holds unchanged.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_batch_exact import F16, NAMES, Q4_0, Q4_K, Q6_K, Q8_0, check_rows, down, up, weights
+
+pytestmark = pytest.mark.gpu
+
+# rows at the edges of 16-row tiles and of the 1, 2 and 4 tiles a workgroup
+# takes; columns at the edges of 16- to 64-column tiles; K of one block, odd
+# block counts (windows straight from memory), one unit of 256, more units
+# than waves, and K split over several workgroups
+CASES = [(Q4_0, 3, 1, 32), (Q4_0, 16, 15, 256), (Q4_0, 17, 16, 288), (Q4_0, 33, 301, 1056), (Q4_0, 64, 4096, 4096),
+         (Q4_0, 20, 1000, 11008), (Q4_0, 130, 100, 2304), (Q4_0, 192, 333, 1024), (Q8_0, 3, 17, 32),
+         (Q8_0, 15, 49, 2080), (Q8_0, 32, 130, 4096), (Q8_0, 63, 64, 544), (Q8_0, 50, 700, 8192), (Q4_K, 4, 3, 256),
+         (Q4_K, 16, 1024, 4096), (Q4_K, 31, 65, 2304), (Q4_K, 65, 500, 14336), (Q6_K, 3, 33, 256),
+         (Q6_K, 16, 47, 768), (Q6_K, 23, 1001, 4096), (Q6_K, 64, 200, 11008), (Q6_K, 100, 129, 2304), (F16, 5, 31, 96),
+         (F16, 16, 129, 4096), (F16, 48, 77, 1056)]
+
+
+@pytest.mark.parametrize("t,M,N,K", CASES, ids=[f"{NAMES[t]}-{m}x{n}x{k}" for t, m, n, k in CASES])
+def test_few_rows(holo, synth, oracle, t, M, N, K):
+    """The product, the add in its store and the SwiGLU in its split: within
+    the bound, the fused forms bit-identical to the unfused sequence, two
+    calls bit-identical, nothing written past the output."""
+    print(f"case few rows {NAMES[t]} {M}x{N}x{K}", flush=True)
+    lib = holo.lib()
+    src, w = weights(synth, oracle, t, N, K, seed=M + 3 * N + K)
+    X = synth.normal(M * K, seed=K + 5).reshape(M, K)
+    U = synth.normal(M * K, seed=K + 6).reshape(M, K)
+    R = synth.normal(M * N, seed=K + 7).reshape(M, N)
+    X[0] *= 1e5  # rows of very different size share a tile
+    X[-1] *= 1e-6
+    dW, dX, dU, dR = up(holo, src), up(holo, X), up(holo, U), up(holo, R)
+    outs = []
+    for _ in range(2):
+        dY = up(holo, np.full(M * N + 64, 7.0, np.float32))
+        lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, t)
+        lib.cuda_sync()
+        holo.check("few rows")
+        outs.append(down(dY, M * N + 64))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    assert np.all(outs[0][M * N:] == 7.0)
+    y = outs[0][:M * N].reshape(M, N)
+    for r in (np.arange(1), np.arange(1, M - 1), np.arange(M - 1, M)):  # each scale by itself
+        if len(r):
+            check_rows(y, X, w, r, t, K)
+    dS, dZ, dG, dH, dT = up(holo, R), up(holo, R), up(holo, X), holo.DeviceBuffer(4 * M * K), holo.DeviceBuffer(4 * M * N)
+    lib.holo_matmul_batch_add(dS.ptr, dW.ptr, dX.ptr, dS.ptr, M, N, K, t)
+    lib.cuda_silu_mul(dH.ptr, dG.ptr, dU.ptr, M * K)
+    lib.holo_matmul_batch(dT.ptr, dW.ptr, dH.ptr, M, N, K, t)
+    lib.holo_matmul_batch_swiglu_add(dZ.ptr, dW.ptr, dG.ptr, dU.ptr, dR.ptr, M, N, K, t)
+    lib.cuda_sync()
+    holo.check("few rows add")
+    assert np.array_equal(down(dS, M * N).reshape(M, N), R + y)
+    assert np.array_equal(down(dZ, M * N).reshape(M, N), R + down(dT, M * N).reshape(M, N))
+
+
+def test_few_rows_multi(holo, synth, oracle):
+    """q, k, v of mixed types and gate, up of one: each output within the bound."""
+    lib = holo.lib()
+    M, K = 23, 2304
+    for types, Ns in (((Q4_K, Q4_K, Q6_K), (256, 128, 128)), ((Q4_0, Q4_0), (384, 384))):
+        srcs, ws = zip(*[weights(synth, oracle, t, n, K, seed=90 + i) for i, (t, n) in enumerate(zip(types, Ns))])
+        X = synth.normal(M * K, seed=91).reshape(M, K)
+        dWs, dX, dYs = [up(holo, s) for s in srcs], up(holo, X), [holo.DeviceBuffer(4 * M * n) for n in Ns]
+        k = len(Ns)
+        lib.holo_matmul_batch_multi_types((C.c_void_p * k)(*[d.ptr for d in dYs]),
+                                          (C.c_void_p * k)(*[d.ptr for d in dWs]), (C.c_int * k)(*types),
+                                          (C.c_int * k)(*Ns), k, dX.ptr, M, K)
+        lib.cuda_sync()
+        holo.check("few rows multi")
+        for i, n in enumerate(Ns):
+            check_rows(down(dYs[i], M * n).reshape(M, n), X, ws[i], np.arange(M), types[i], K)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 512, 2048), (40, 2000, 11008)], ids=["whole", "parts"])
+def test_few_rows_streams_and_graph(holo, synth, oracle, M, N, K):
+    """Calls issued on two streams at once, and a captured graph replayed
+    between eager calls: the bits of the call on its own."""
+    lib = holo.lib()
+    src, _ = weights(synth, oracle, Q4_0, N, K, seed=N)
+    Xs = [synth.normal(M * K, seed=s).reshape(M, K) for s in (1, 2)]
+    dW, dXs = up(holo, src), [up(holo, x) for x in Xs]
+
+    def call(x):
+        d = holo.DeviceBuffer(4 * M * N)
+        lib.holo_matmul_batch(d.ptr, dW.ptr, x.ptr, M, N, K, Q4_0)
+        return d
+
+    want = [call(x) for x in dXs]
+    lib.cuda_sync()
+    want = [down(d, M * N).view(np.uint32) for d in want]
+    streams = [lib.holo_stream_create() for _ in range(2)]
+    try:
+        got = []
+        for _ in range(6):
+            for s, x in zip(streams, dXs):
+                lib.holo_set_stream(s)
+                got.append(call(x))
+        lib.cuda_sync()
+        for i, d in enumerate(got):
+            assert np.array_equal(down(d, M * N).view(np.uint32), want[i % 2]), i
+        dG = holo.DeviceBuffer(4 * M * N)
+        lib.holo_set_stream(streams[0])
+        assert lib.holo_graph_begin() == 0
+        lib.holo_matmul_batch(dG.ptr, dW.ptr, dXs[0].ptr, M, N, K, Q4_0)
+        g = lib.holo_graph_end()
+        holo.check("capture")
+        for rep in range(3):
+            lib.holo_graph_launch(g)
+            other = call(dXs[1])
+            lib.cuda_sync()
+            assert np.array_equal(down(dG, M * N).view(np.uint32), want[0]), rep
+            assert np.array_equal(down(other, M * N).view(np.uint32), want[1]), rep
+        lib.holo_graph_destroy(g)
+    finally:
+        lib.holo_set_stream(None)
+        for s in streams:
+            lib.holo_stream_destroy(s)
+    holo.check("streams")
+
+
+def test_few_rows_keeps_gemv_cases(holo, synth, oracle):
+    """Rows that the product does not take still run one GEMV each: no matrix
+    (zeros), another activation mode, activations off 16-byte alignment."""
+    lib = holo.lib()
+    M, N, K = 5, 70, 512
+    src, _ = weights(synth, oracle, Q4_0, N, K, seed=4)
+    X = synth.normal(M * K + 1, seed=5)
+    dW, dX, dY = up(holo, src), up(holo, X), up(holo, np.ones(M * N, np.float32))
+    lib.holo_matmul_rows(dY.ptr, None, dX.ptr, M, N, K, Q4_0, 0)
+    lib.cuda_sync()
+    holo.check("no matrix")
+    assert np.all(down(dY, M * N) == 0)
+    ref = np.stack([oracle.matmul(Q4_0, src, X[1 + m * K:1 + (m + 1) * K], N, K) for m in range(M)])
+    lib.holo_matmul_rows(dY.ptr, dW.ptr, dX.ptr + 4, M, N, K, Q4_0, 0)
+    lib.cuda_sync()
+    holo.check("misaligned rows")
+    assert np.max(np.abs(down(dY, M * N).reshape(M, N) - ref)) <= 1e-3 * np.max(np.abs(ref))
+    single = holo.DeviceBuffer(4 * N)
+    lib.holo_gemv_set_xmode(0)
+    try:
+        lib.holo_matmul_rows(dY.ptr, dW.ptr, dX.ptr, M, N, K, Q4_0, 0)
+        lib.holo_matmul(single.ptr, dW.ptr, dX.ptr + 4 * K, N, K, Q4_0)
+        lib.cuda_sync()
+    finally:
+        lib.holo_gemv_set_xmode(2)
+    holo.check("fp32 mode")
+    assert np.array_equal(down(dY, M * N).reshape(M, N)[1], down(single, N))
+
+
+def test_few_rows_infinities(holo, synth, oracle):
+    """A row with an infinity gives infinities and NaNs, as fp32 does; the
+    other rows keep their bits."""
+    lib = holo.lib()
+    M, N, K = 7, 40, 512
+    src, w = weights(synth, oracle, Q8_0, N, K, seed=14)
+    X = synth.normal(M * K, seed=15).reshape(M, K)
+    dW, outs = up(holo, src), []
+    for k in range(2):
+        if k:
+            X[3, 100] = np.inf
+        dX, dY = up(holo, X), holo.DeviceBuffer(4 * M * N)
+        lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, Q8_0)
+        lib.cuda_sync()
+        outs.append(down(dY, M * N).reshape(M, N))
+    holo.check("infinities")
+    rest = np.r_[0:3, 4:7]
+    assert np.array_equal(outs[0][rest], outs[1][rest])
+    want = np.where(w[:, 100] > 0, np.inf, np.where(w[:, 100] < 0, -np.inf, np.nan))
+    assert np.array_equal(outs[1][3], want, equal_nan=True)
