@@ -33,6 +33,12 @@ void gemv_stream_release();
 // without them decode attention runs one range per head.
 bool attention_scratch_init();
 void attention_scratch_release();
+// A decode step's attention with its RoPE, for rows that fit it: q and the raw
+// key kx of position pos are rotated on the way in and the key's cache row is
+// written (the value's is there already).
+bool attention_decode_fits(const float *q, const float *kc, const float *vc, int hd);
+void attention_decode_rope(float *dst, const float *q, const float *kx, float *kc, const float *vc, int pos, int hd,
+                           int n_heads, int n_kv_heads, float base);
 void panel_workspace_release();  // the batched products' panel buffers (prefill.hip)
 // The batched products' kept workspaces (prefill.hip): slot 0 weight panels,
 // slot 1 activation panels, slot 2 the exact product's split-K partials.  A device buffer of at least `bytes`, grown with

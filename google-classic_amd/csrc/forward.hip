@@ -177,11 +177,12 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
     const int exact = flags & HOLO_FORWARD_EXACT;
     const int64_t layer_cache = (int64_t)m->max_seq * kv_dim;
 
-    // stream-ordered scratch: token ids, x, xb, q, att, hb, hb2 (k and v are
-    // written straight into the caches)
+    // stream-ordered scratch: token ids, x, xb, q, att, hb, hb2, and one raw key
+    // row (otherwise k and v are written straight into the caches)
     const size_t rowsz = (size_t)n * sizeof(float);
     const size_t sz_tok = ((size_t)n * sizeof(int) + 255) & ~(size_t)255;
-    const size_t sizes[] = {sz_tok, rowsz * dim, rowsz * dim, rowsz * q_dim, rowsz * q_dim, rowsz * ffn, rowsz * ffn};
+    const size_t sizes[] = {sz_tok, rowsz * dim, rowsz * dim, rowsz * q_dim, rowsz * q_dim, rowsz * ffn, rowsz * ffn,
+                            sizeof(float) * (size_t)kv_dim};
     constexpr int kBufs = sizeof(sizes) / sizeof(sizes[0]);
     size_t total = 0;
     for (size_t s : sizes) total += (s + 255) & ~(size_t)255;
@@ -197,6 +198,7 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
     int *dtok = (int *)bufs[0];
     float *x = (float *)bufs[1], *xb = (float *)bufs[2], *q = (float *)bufs[3], *att = (float *)bufs[4];
     float *hb = (float *)bufs[5], *hb2 = (float *)bufs[6];
+    float *kx = (float *)bufs[7];
 
     // embeddings: all n rows in one launch
     HOLO_CHECK(hipMemcpyAsync(dtok, tokens, (size_t)n * sizeof(int), hipMemcpyHostToDevice, stream()));
@@ -207,10 +209,14 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
         float *kc = m->key_cache + l * layer_cache, *vc = m->value_cache + l * layer_cache;
         // this call's rows of the caches: the k and v products land there
         // directly ([pos][kv_dim] is their row-major output layout)
-        float *k = kc + (int64_t)pos0 * kv_dim, *v = vc + (int64_t)pos0 * kv_dim;
+        float *kr = kc + (int64_t)pos0 * kv_dim, *v = vc + (int64_t)pos0 * kv_dim;
         // One row (a decode step): the norms run inside the q/k/v and gate/up
         // GEMVs and the residual adds inside the o and down GEMVs.
         const bool one = n == 1;
+        // The attention of one row rotates q and k itself: k goes to scratch,
+        // its rotated row into the cache from there.
+        const bool rope1 = one && attention_decode_fits(q, kc, vc, hd);
+        float *k = rope1 ? kx : kr;
         const bool qkv1 = one && L.attn_norm && fused_gemv_type(L.wq_type) && L.wk_type == L.wq_type &&
                           L.wv_type == L.wq_type;
         const bool ffn1 = one && L.ffn_norm && fused_gemv_type(L.w1_type) && L.w3_type == L.w1_type;
@@ -222,8 +228,12 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
             norm_or_copy(xb, x, L.attn_norm, n, dim, m->rms_eps);
             matmul_qkv(q, k, v, L, xb, n, q_dim, kv_dim, dim, exact);
         }
-        holo_rope_rows(q, k, n, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base);  // k rotated in the cache
-        holo_attention_prefill(att, q, kc, vc, n, pos0, hd, m->n_heads, m->n_kv_heads);
+        if (rope1) {
+            attention_decode_rope(att, q, kx, kc, vc, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base);
+        } else {
+            holo_rope_rows(q, k, n, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base);  // k rotated in the cache
+            holo_attention_prefill(att, q, kc, vc, n, pos0, hd, m->n_heads, m->n_kv_heads);
+        }
         if (one && fused_gemv_type(L.wo_type)) {
             holo_matmul_add(x, L.wo, att, x, dim, q_dim, L.wo_type);
         } else if (gemm_rows(L.wo_type, n, q_dim, exact)) {

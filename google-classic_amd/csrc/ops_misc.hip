@@ -612,291 +612,284 @@ static int q6_rows_per_wave(int out_dim)
 // cuda_multi_head_attention computes it (cuda_ops.cu:1813-1952), for heads of
 // up to 128 dims (a multiple of 4).  The keys are cut into `splits` ranges of
 // `chunk` positions, one workgroup per (range, head), so that a decode step
-// reads the whole cache with the whole chip rather than one workgroup per head.
-// A workgroup takes its range 64 positions at a time: thread (c, g) owns
-// 16-byte column c of the head (32 columns) for keys g, g + 8, ..., g + 56, so
-// all 8 key and 8 value loads of a thread are issued together and each wave
-// instruction reads two whole 512-byte cache rows.  Scores are summed over the
-// 32 column lanes, the softmax runs online over the 64-key passes (running
-// max and sum), and the 8 key groups' partial outputs are summed in a fixed
-// order.  With one range the workgroup writes the output; otherwise it writes
-// (unnormalised output, max, sum) and attn_decode_combine_k merges the ranges
-// of a head in range order, so the result does not depend on timing.
-constexpr int kDecKeys = 64;
-constexpr int kDecMaxSplits = 256;  // at most one range per thread of attn_decode_combine_k's 512
+// reads the cache with the whole chip rather than one workgroup per head.
+// With one range the workgroup writes the output; otherwise it writes
+// (unnormalised output, max, sum), and attn_dec_merge_k merges the ranges of a
+// head in range order, so the result does not depend on timing.
+//
+// Within a range the softmax state is kept per key group: groups of LPK lanes
+// (a head's 16-byte columns) take every G-th key, J at a time, and hold their
+// own running max, sum and output; nothing crosses the groups until the end,
+// where they meet in group order.  (Workgroup-wide scores, max and sum for
+// every 64 keys cost two barriers and a dozen cross-lane steps a pass.)  Two
+// passes' keys and values are in flight.  Scores are in log2 units (q scaled by
+// log2(e) / sqrt(hd)).
+//
+// What bounds it: at 2048 positions of 32 heads the cache read (67 MB), 13.7
+// us in all against 13.3 at a large copy's rate and 19.7 before; at 512 the
+// launches and one round trip of loads (range kernel 6.4, merge 2.4 us; before
+// 8.8 and 4.0).
 constexpr size_t kDecPartFloats = (size_t)4 << 20;  // 16 MiB of range partials, allocated by cuda_init
 static float *g_dec_part = nullptr;
+constexpr int kDecThreads = 512;
+constexpr int kDecMaxSplits = 256;
 
-__device__ __forceinline__ float half_wave_sum(float v)
+// Merges a head's ranges with weights 2^(m_s - M), NS of them per round of
+// loads: thread d holds every range's output d, max and sum, so nothing is
+// exchanged and a merge of up to NS ranges waits once.
+template <int NS>
+__global__ __launch_bounds__(128) void attn_dec_merge_k(float *out, const float *part, int hd, int splits)
 {
+    const int h = blockIdx.x, d = threadIdx.x, stride = hd + 4;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(part + (int64_t)h * splits * stride), (short)0, splits * stride * 4, kRawBufWord3);
+    float M = -INFINITY, L = 0.f, a = 0.f;
+    for (int s0 = 0; s0 < splits; s0 += NS) {
+        float o[NS], m[NS], l[NS];
 #pragma unroll
-    for (int off = 1; off < 32; off <<= 1) v += __shfl_xor(v, off, 32);
+        for (int s = 0; s < NS; s++) {  // ranges past the last read zeros
+            const int so = 4 * (s0 + s) * stride;
+            o[s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, 4 * d, so, 0));
+            const auto ml = __builtin_amdgcn_raw_buffer_load_b64(r, 4 * hd, so, 0);
+            m[s] = s0 + s < splits ? __uint_as_float(ml[0]) : -INFINITY;
+            l[s] = __uint_as_float(ml[1]);
+        }
+        float mx = fmaxf(M, m[0]);
+#pragma unroll
+        for (int s = 1; s < NS; s++) mx = fmaxf(mx, m[s]);
+        const float c = __builtin_amdgcn_exp2f(M - mx);  // 0 in the first round
+        L *= c;
+        a *= c;
+        M = mx;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const float w = __builtin_amdgcn_exp2f(m[s] - M);
+            L = fmaf(w, l[s], L);
+            a = fmaf(w, o[s], a);
+        }
+    }
+    if (d < hd) out[(int64_t)h * hd + d] = a * (1.0f / L);
+}
+
+// ROPE (a decode step's attention with its rotation): q and the new key (raw,
+// kx) are rotated here, with rope_head's expressions, while the first cache
+// rows are on their way; the new position is the last one, its key comes from
+// LDS, and the first head of a KV head writes it to the cache.
+struct DecArgs {
+    float *out, *part;
+    const float *q, *kc, *vc;
+    const float *kx;  // ROPE: [n_kv_heads * hd], the raw key of position kv_len - 1
+    float *kw;        // ROPE: its cache row
+    int kv_len, hd, n_heads, n_kv_heads, chunk;
+    float base;
+};
+
+// Sum over the LPK (16 or 32) lanes of a group, in every lane.
+template <int LPK>
+__device__ __forceinline__ float group_sum(float v)
+{
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));   // quad [1,0,3,2]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));   // quad [2,3,0,1]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));  // half mirror
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));  // mirror
+    if constexpr (LPK == 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
     return v;
 }
 
-__global__ __launch_bounds__(256) void attn_decode_k(float *out, float *part, const float *q, const float *kc,
-                                                     const float *vc, int kv_len, int hd, int n_heads, int n_kv_heads,
-                                                     int chunk)
+template <int LPK, bool ROPE>
+__global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
 {
-    __shared__ float4 lq[32];
-    __shared__ float lsc[kDecKeys];
-    __shared__ float4 lo[8][32];
-    const int h = blockIdx.y, s = blockIdx.x, splits = gridDim.x;
-    const int kvh = h / (n_heads / n_kv_heads);
-    const int64_t kv_dim = (int64_t)n_kv_heads * hd;
-    const int t = threadIdx.x, lane = t & 63, c = t & 31, g = t >> 5;
+    constexpr int G = kDecThreads / LPK, J = 4, W = kDecThreads / 64;
+    __shared__ __align__(16) float lq[128], lk[128];
+    __shared__ float lo[W][128];
+    __shared__ float lm[W], ll[W];
+    const int h = blockIdx.y, s = blockIdx.x, splits = gridDim.x, hd = a.hd;
+    const int kvh = h / (a.n_heads / a.n_kv_heads);
+    const int64_t kv_dim = (int64_t)a.n_kv_heads * hd;
+    const int t = threadIdx.x, c = t & (LPK - 1), g = t / LPK;
     const int hd4 = hd >> 2;
     const bool col = c < hd4;
-    const float scale = 1.0f / sqrtf((float)hd);
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < hd4) lq[t] = *(const float4 *)(q + (int64_t)h * hd + 4 * t);
+    const int p_begin = s * a.chunk, p_end = min(p_begin + a.chunk, a.kv_len);
+    const float *kb = a.kc + (int64_t)kvh * hd, *vb = a.vc + (int64_t)kvh * hd;
+    // through buffer resources from each pass's first key: keys past the range
+    // and lanes past the head read zeros, without branches
+    const uint32_t rowb = (uint32_t)kv_dim * 4u;
+    const uint32_t vo = col ? (uint32_t)g * rowb + 16u * (uint32_t)c : 0x80000000u;
+    float4 k4[2][J], v4[2][J];
+    auto load = [&](int b, int p0) {
+        const int64_t left = p0 < p_end ? ((int64_t)(p_end - p0 - 1) * kv_dim + hd) * 4 : 0;
+        const int bytes = (int)min(left, (int64_t)0x7FFFFFFF);
+        const int64_t at = (int64_t)min(p0, p_end - 1) * kv_dim;
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(kb + at), (short)0, bytes, kRawBufWord3);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vb + at), (short)0, bytes, kRawBufWord3);
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            k4[b][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)vo, (int)((uint32_t)(G * j) * rowb), 0));
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            v4[b][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, (int)vo, (int)((uint32_t)(G * j) * rowb), 0));
+    };
+    load(0, p_begin);
+    load(1, p_begin + G * J);
+    const float scale = 1.4426950408889634f / sqrtf((float)hd);
+    const bool last = ROPE && p_end == a.kv_len;  // this range holds the new position
+    if constexpr (ROPE) {
+        // one pair per thread: q's first, then the key's
+        const int half = hd / 2, i = t < half ? t : t - half;
+        if (t < (last ? hd : half)) {
+            const float freq = 1.0f / powf(a.base, (float)(2 * i) / (float)hd);
+            const float th = (float)(a.kv_len - 1) * freq;
+            const float cs = cosf(th), sn = sinf(th);
+            const float *src = t < half ? a.q + (int64_t)h * hd : a.kx + (int64_t)kvh * hd;
+            float *dst = t < half ? lq : lk;
+            const float x = src[i], y = src[i + half];
+            dst[i] = x * cs - y * sn;
+            dst[i + half] = x * sn + y * cs;
+        }
+    } else {
+        if (t < hd4) *(float4 *)(lq + 4 * t) = *(const float4 *)(a.q + (int64_t)h * hd + 4 * t);
+    }
     __syncthreads();
-    const float4 q4 = col ? lq[c] : zero;
-    const float *kb = kc + (int64_t)kvh * hd + 4 * c;
-    const float *vb = vc + (int64_t)kvh * hd + 4 * c;
-    const int p_begin = s * chunk, p_end = min(p_begin + chunk, kv_len);
-    float m = -INFINITY, l = 0.f;
+    const float4 q0 = col ? *(const float4 *)(lq + 4 * c) : zero;
+    const float4 q4 = make_float4(q0.x * scale, q0.y * scale, q0.z * scale, q0.w * scale);
+    float4 kn = zero;
+    if (last && col) {
+        kn = *(const float4 *)(lk + 4 * c);
+        if (g == 0 && h % (a.n_heads / a.n_kv_heads) == 0) *(float4 *)(a.kw + (int64_t)kvh * hd + 4 * c) = kn;
+    }
+    float m = -1e30f, l = 0.f;
     float4 o4 = zero;
-    for (int p0 = p_begin; p0 < p_end; p0 += kDecKeys) {
-        float4 k4[8], v4[8];
+    auto use = [&](int b, int p0) {
+        float sj[J];
+        float mx = m;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int p = p0 + g + 8 * j;
-            k4[j] = zero;
-            v4[j] = zero;
-            if (col && p < p_end) {
-                k4[j] = *(const float4 *)(kb + (int64_t)p * kv_dim);
-                v4[j] = *(const float4 *)(vb + (int64_t)p * kv_dim);
-            }
+        for (int j = 0; j < J; j++) {
+            const int p = p0 + g + G * j;
+            float4 k = k4[b][j];
+            if (ROPE && p == a.kv_len - 1) k = kn;
+            const float d = group_sum<LPK>(q4.x * k.x + q4.y * k.y + q4.z * k.z + q4.w * k.w);
+            sj[j] = p < p_end ? d : -INFINITY;
+            mx = fmaxf(mx, sj[j]);
         }
-        float sj[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            sj[j] = half_wave_sum(q4.x * k4[j].x + q4.y * k4[j].y + q4.z * k4[j].z + q4.w * k4[j].w);
-        if (c == 0) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) lsc[g + 8 * j] = p0 + g + 8 * j < p_end ? sj[j] * scale : -INFINITY;
-        }
-        __syncthreads();
-        // every wave reduces the same 64 scores in the same order, so m and l
-        // agree across the workgroup; key p0 + i's weight sits in lane i
-        const float sl = lsc[lane];
-        const float mnew = fmaxf(m, wave_reduce_max(sl));  // p0 < p_end: finite from the first pass on
-        const float corr = expf(m - mnew);
-        const float pl = expf(sl - mnew);
-        l = l * corr + wave_reduce_sum(pl);
+        const float corr = __builtin_amdgcn_exp2f(m - mx);
+        m = mx;
+        l *= corr;
         o4 = make_float4(o4.x * corr, o4.y * corr, o4.z * corr, o4.w * corr);
-        m = mnew;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float w = __shfl(pl, g + 8 * j, 64);
-            o4 = make_float4(fmaf(w, v4[j].x, o4.x), fmaf(w, v4[j].y, o4.y), fmaf(w, v4[j].z, o4.z),
-                             fmaf(w, v4[j].w, o4.w));
+        for (int j = 0; j < J; j++) {
+            const float w = __builtin_amdgcn_exp2f(sj[j] - m);
+            l += w;
+            o4 = make_float4(fmaf(w, v4[b][j].x, o4.x), fmaf(w, v4[b][j].y, o4.y), fmaf(w, v4[b][j].z, o4.z),
+                             fmaf(w, v4[b][j].w, o4.w));
         }
-        __syncthreads();  // lsc is rewritten by the next pass
+    };
+    for (int p0 = p_begin; p0 < p_end; p0 += 2 * G * J) {
+        use(0, p0);
+        load(0, p0 + 2 * G * J);
+        use(1, p0 + G * J);
+        load(1, p0 + 3 * G * J);
     }
-    lo[g][c] = o4;
-    __syncthreads();
-    if (t < hd4) {
-        float4 r = lo[0][t];
+    // the groups of a wave first (64 / LPK of them), then the waves through LDS
 #pragma unroll
-        for (int gg = 1; gg < 8; gg++)
-            r = make_float4(r.x + lo[gg][t].x, r.y + lo[gg][t].y, r.z + lo[gg][t].z, r.w + lo[gg][t].w);
-        if (splits == 1) {
-            const float inv = 1.0f / l;
-            *(float4 *)(out + (int64_t)h * hd + 4 * t) = make_float4(r.x * inv, r.y * inv, r.z * inv, r.w * inv);
-        } else {
-            float *pp = part + ((int64_t)h * splits + s) * (hd + 4);
-            *(float4 *)(pp + 4 * t) = r;
-            if (t == 0) {
-                pp[hd] = m;
-                pp[hd + 1] = l;
-            }
-        }
+    for (int off = 32; off >= LPK; off >>= 1) {
+        const float m2 = __shfl_xor(m, off, 64), l2 = __shfl_xor(l, off, 64);
+        const float mx = fmaxf(m, m2), w1 = __builtin_amdgcn_exp2f(m - mx), w2 = __builtin_amdgcn_exp2f(m2 - mx);
+        const float4 r = make_float4(__shfl_xor(o4.x, off, 64), __shfl_xor(o4.y, off, 64), __shfl_xor(o4.z, off, 64),
+                                     __shfl_xor(o4.w, off, 64));
+        o4 = make_float4(w1 * o4.x + w2 * r.x, w1 * o4.y + w2 * r.y, w1 * o4.z + w2 * r.z, w1 * o4.w + w2 * r.w);
+        l = w1 * l + w2 * l2;
+        m = mx;
     }
-}
-
-// Merges a head's ranges with weights e^(m_s - M).  512 threads: thread
-// (d, g) sums ranges g, g + 4, ... for output dim d, and the 4 groups' sums
-// meet in LDS in group order, so the order is fixed.  (Merging in the split
-// kernel itself, by the last range of a head to arrive, measured slower: the
-// merge becomes a serial tail and every range pays the arrival.)
-static_assert(kDecMaxSplits <= 512, "attn_decode_combine_k: one range per thread");
-__global__ __launch_bounds__(512) void attn_decode_combine_k(float *out, const float *part, int hd, int splits)
-{
-    __shared__ float lw[kDecMaxSplits];
-    __shared__ float lg[4][128];
-    __shared__ float scratch[16];
-    const int h = blockIdx.x, t = threadIdx.x, d = t & 127, grp = t >> 7;
-    const int stride = hd + 4;
-    const float *ph = part + (int64_t)h * splits * stride;
-    // one round of loads: the partial outputs of ranges grp, grp + 4, ... (the
-    // first kPre of them into registers) together with range t's max and sum,
-    // so the reductions below wait for a single round trip
-    constexpr int kPre = 16;
-    float po[kPre];
-#pragma unroll
-    for (int i = 0; i < kPre; i++) {
-        const int s = grp + 4 * i;
-        po[i] = d < hd && s < splits ? ph[(int64_t)s * stride + d] : 0.f;
-    }
-    const bool mine = t < splits;  // splits <= kDecMaxSplits <= blockDim.x: one range per thread at most
-    const float ms = mine ? ph[(int64_t)t * stride + hd] : -INFINITY;
-    const float ls = mine ? ph[(int64_t)t * stride + hd + 1] : 0.f;
-    const float M = block_reduce<true>(ms, scratch);
-    const float w = mine ? expf(ms - M) : 0.f;
-    if (mine) lw[t] = w;
-    const float L = block_reduce<false>(w * ls, scratch);  // its barriers also publish lw
-    if (d < hd) {
-        float o = 0.f;
-#pragma unroll
-        for (int i = 0; i < kPre; i++)
-            if (grp + 4 * i < splits) o = fmaf(lw[grp + 4 * i], po[i], o);
-        for (int s = grp + 4 * kPre; s < splits; s += 4) o = fmaf(lw[s], ph[(int64_t)s * stride + d], o);
-        lg[grp][d] = o;
+    const int wave = t >> 6;
+    if ((t & 63) < LPK && col) *(float4 *)(&lo[wave][4 * c]) = o4;
+    if ((t & 63) == 0) {
+        lm[wave] = m;
+        ll[wave] = l;
     }
     __syncthreads();
-    if (grp == 0 && d < hd) out[(int64_t)h * hd + d] = (((lg[0][d] + lg[1][d]) + lg[2][d]) + lg[3][d]) * (1.0f / L);
-}
-
-// Short caches in one launch: one workgroup per head, SUB groups of 256
-// threads, group sg taking positions [sg chunk, (sg + 1) chunk) with
-// attn_decode_k's pass (the same loads, scores, online softmax and key-group
-// order), every group looping the same number of passes so the barriers are
-// the workgroup's.  A group whose range is empty keeps (m, l, o) = (-inf, 0,
-// 0) and gets weight 0; the groups merge in group order through LDS, so the
-// result does not depend on timing.  No range partials and no second launch.
-template <int SUB>
-__global__ __launch_bounds__(256 * SUB) void attn_decode_wg_k(float *out, const float *q, const float *kc,
-                                                              const float *vc, int kv_len, int hd, int n_heads,
-                                                              int n_kv_heads, int chunk)
-{
-    __shared__ float4 lq[32];
-    __shared__ float lsc[SUB][kDecKeys];
-    __shared__ float4 lo[SUB][8][32];
-    __shared__ float lm[SUB], ll[SUB];
-    const int h = blockIdx.x;
-    const int kvh = h / (n_heads / n_kv_heads);
-    const int64_t kv_dim = (int64_t)n_kv_heads * hd;
-    const int t = threadIdx.x, sg = __builtin_amdgcn_readfirstlane(t >> 8), u = t & 255;
-    const int lane = u & 63, c = u & 31, g = u >> 5;
-    const int hd4 = hd >> 2;
-    const bool col = c < hd4;
-    const float scale = 1.0f / sqrtf((float)hd);
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < hd4) lq[t] = *(const float4 *)(q + (int64_t)h * hd + 4 * t);
-    __syncthreads();
-    const float4 q4 = col ? lq[c] : zero;
-    const float *kb = kc + (int64_t)kvh * hd + 4 * c;
-    const float *vb = vc + (int64_t)kvh * hd + 4 * c;
-    const int p_begin = sg * chunk, p_end = min(p_begin + chunk, kv_len);
-    float m = -INFINITY, l = 0.f;
-    float4 o4 = zero;
-    for (int i0 = 0; i0 < chunk; i0 += kDecKeys) {
-        const int p0 = p_begin + i0;
-        float4 k4[8], v4[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int p = p0 + g + 8 * j;
-            k4[j] = zero;
-            v4[j] = zero;
-            if (col && p < p_end) {
-                k4[j] = *(const float4 *)(kb + (int64_t)p * kv_dim);
-                v4[j] = *(const float4 *)(vb + (int64_t)p * kv_dim);
-            }
-        }
-        float sj[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            sj[j] = half_wave_sum(q4.x * k4[j].x + q4.y * k4[j].y + q4.z * k4[j].z + q4.w * k4[j].w);
-        if (c == 0) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) lsc[sg][g + 8 * j] = p0 + g + 8 * j < p_end ? sj[j] * scale : -INFINITY;
-        }
-        __syncthreads();
-        if (p0 < p_end) {  // uniform per group: a pass with keys in this group's range
-            const float sl = lsc[sg][lane];
-            const float mnew = fmaxf(m, wave_reduce_max(sl));  // finite: the pass has a key
-            const float corr = expf(m - mnew);
-            const float pl = expf(sl - mnew);
-            l = l * corr + wave_reduce_sum(pl);
-            o4 = make_float4(o4.x * corr, o4.y * corr, o4.z * corr, o4.w * corr);
-            m = mnew;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float w = __shfl(pl, g + 8 * j, 64);
-                o4 = make_float4(fmaf(w, v4[j].x, o4.x), fmaf(w, v4[j].y, o4.y), fmaf(w, v4[j].z, o4.z),
-                                 fmaf(w, v4[j].w, o4.w));
-            }
-        }
-        __syncthreads();  // lsc is rewritten by the next pass
-    }
-    lo[sg][g][c] = o4;
-    if (u == 0) {
-        lm[sg] = m;
-        ll[sg] = l;
-    }
-    __syncthreads();
-    if (t < hd4) {
+    if (t < hd) {
         float M = lm[0];
 #pragma unroll
-        for (int k = 1; k < SUB; k++) M = fmaxf(M, lm[k]);  // group 0 always has keys: finite
-        float L = 0.f;
-        float4 r = zero;
+        for (int w = 1; w < W; w++) M = fmaxf(M, lm[w]);
+        float L = 0.f, r = 0.f;
 #pragma unroll
-        for (int k = 0; k < SUB; k++) {
-            const float w = lm[k] == -INFINITY ? 0.f : expf(lm[k] - M);
-            float4 rk = lo[k][0][t];
-#pragma unroll
-            for (int gg = 1; gg < 8; gg++)
-                rk = make_float4(rk.x + lo[k][gg][t].x, rk.y + lo[k][gg][t].y, rk.z + lo[k][gg][t].z,
-                                 rk.w + lo[k][gg][t].w);
-            r = make_float4(fmaf(w, rk.x, r.x), fmaf(w, rk.y, r.y), fmaf(w, rk.z, r.z), fmaf(w, rk.w, r.w));
-            L = fmaf(w, ll[k], L);
+        for (int w = 0; w < W; w++) {
+            const float e = __builtin_amdgcn_exp2f(lm[w] - M);
+            L = fmaf(e, ll[w], L);
+            r = fmaf(e, lo[w][t], r);
         }
-        const float inv = 1.0f / L;
-        *(float4 *)(out + (int64_t)h * hd + 4 * t) = make_float4(r.x * inv, r.y * inv, r.z * inv, r.w * inv);
+        if (splits == 1) {
+            a.out[(int64_t)h * hd + t] = r * (1.0f / L);
+        } else {
+            float *pp = a.part + ((int64_t)h * splits + s) * (hd + 4);
+            pp[t] = r;
+            if (t == 0) {
+                pp[hd] = M;
+                pp[hd + 1] = L;
+            }
+        }
     }
 }
-// Up to this many positions (one 64-position pass per group) attn_decode_wg_k:
-// 6.6 against 8.0 us at 128 positions, 32 heads of 128.  With two or more
-// passes its 32 workgroups wait on each pass in turn, and the split kernel's
-// whole-chip read wins (300 / 512 / 1024 positions: 9.8 / 10.8 / 19.4 against
-// 8.3 / 8.5 / 10.1 us).
-constexpr int kDecWgMaxKeys = 4 * kDecKeys;
 
-// Shapes the split kernel takes: head_dim a multiple of 4 up to 128, 16-byte
+// Shapes the kernel above takes: head_dim a multiple of 4 up to 128, 16-byte
 // aligned rows.
-static bool decode_attention_fits(const float *q, const float *kc, const float *vc, int hd)
+bool attention_decode_fits(const float *q, const float *kc, const float *vc, int hd)
 {
     return hd >= 4 && hd <= 128 && hd % 4 == 0 && !(((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15);
+}
+
+// Ranges of a call: one where the whole cache fits two passes of one
+// workgroup (256 positions of 128: 5.2 us in one launch, 7.0 in two; 400:
+// 8.2 / 7.1), else about one workgroup per CU, of at least 64 positions (1024
+// positions x 32 heads: 8 ranges 9.5 us, 4 12.1, 16 10.8), and no more than
+// 16 per head where there are half as many workgroups anyway (2805 positions
+// x 8 heads: 15 ranges 6.7 us, 30 8.4).
+static int decode_splits(int kv_len, int hd, int n_heads)
+{
+    if (!g_dec_part || (int64_t)kv_len * hd <= 256 * 128) return 1;
+    int want = num_cus() / n_heads;
+    if (want > 16) want = max(16, num_cus() / 2 / n_heads);
+    want = min(want, min(kDecMaxSplits, (int)(kDecPartFloats / ((size_t)n_heads * (hd + 4)))));
+    return max(1, min(want, (kv_len + 63) / 64));
+}
+
+static void decode_attention(DecArgs a, bool rope)
+{
+    int splits = decode_splits(a.kv_len, a.hd, a.n_heads);
+    a.chunk = (a.kv_len + splits - 1) / splits;
+    splits = (a.kv_len + a.chunk - 1) / a.chunk;  // every range holds at least one key
+    a.part = g_dec_part;
+    auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(splits, a.n_heads), dim3(kDecThreads), 0, stream(), a);
+    };
+    if (rope) a.hd > 64 ? run(attn_dec_k<32, true>) : run(attn_dec_k<16, true>);
+    else a.hd > 64 ? run(attn_dec_k<32, false>) : run(attn_dec_k<16, false>);
+    HOLO_LAUNCH_CHECK();
+    if (splits > 1) {
+        if (splits <= 8)
+            hipLaunchKernelGGL(attn_dec_merge_k<8>, dim3(a.n_heads), dim3(128), 0, stream(), a.out, a.part, a.hd, splits);
+        else
+            hipLaunchKernelGGL(attn_dec_merge_k<16>, dim3(a.n_heads), dim3(128), 0, stream(), a.out, a.part, a.hd, splits);
+        HOLO_LAUNCH_CHECK();
+    }
 }
 
 static void decode_attention(float *dst, const float *q, const float *kc, const float *vc, int kv_len, int hd,
                              int n_heads, int n_kv_heads)
 {
-    if (kv_len > kDecKeys && kv_len <= kDecWgMaxKeys) {
-        // four groups of whole 64-position passes per head
-        const int chunk = ((kv_len + 3) / 4 + kDecKeys - 1) / kDecKeys * kDecKeys;
-        hipLaunchKernelGGL(attn_decode_wg_k<4>, dim3(n_heads), dim3(1024), 0, stream(), dst, q, kc, vc, kv_len, hd,
-                           n_heads, n_kv_heads, chunk);
-        HOLO_LAUNCH_CHECK();
-        return;
-    }
-    int splits = (kv_len + kDecKeys - 1) / kDecKeys;
-    if (!g_dec_part) splits = 1;
-    splits = min(splits, min(kDecMaxSplits, (int)(kDecPartFloats / ((size_t)n_heads * (hd + 4)))));
-    splits = max(splits, 1);
-    const int chunk = ((kv_len + splits - 1) / splits + kDecKeys - 1) / kDecKeys * kDecKeys;
-    splits = (kv_len + chunk - 1) / chunk;  // every range holds at least one key
-    hipLaunchKernelGGL(attn_decode_k, dim3(splits, n_heads), dim3(256), 0, stream(), dst, g_dec_part, q, kc, vc,
-                       kv_len, hd, n_heads, n_kv_heads, chunk);
-    HOLO_LAUNCH_CHECK();
-    if (splits > 1) {
-        hipLaunchKernelGGL(attn_decode_combine_k, dim3(n_heads), dim3(512), 0, stream(), dst, g_dec_part, hd,
-                           splits);
-        HOLO_LAUNCH_CHECK();
-    }
+    decode_attention(DecArgs{dst, nullptr, q, kc, vc, nullptr, nullptr, kv_len, hd, n_heads, n_kv_heads, 0, 0.f}, false);
+}
+
+void attention_decode_rope(float *dst, const float *q, const float *kx, float *kc, const float *vc, int pos, int hd,
+                           int n_heads, int n_kv_heads, float base)
+{
+    decode_attention(DecArgs{dst, nullptr, q, kc, vc, kx, kc + (int64_t)pos * n_kv_heads * hd, pos + 1, hd, n_heads,
+                             n_kv_heads, 0, base},
+                     true);
 }
 
 bool attention_scratch_init()
@@ -1476,7 +1469,7 @@ void cuda_multi_head_attention(float *dst, const float *q, const float *k_cache,
         HOLO_REJECT("cuda_multi_head_attention: null pointer or n_heads not a multiple of n_kv_heads");
         return;
     }
-    if (decode_attention_fits(q, k_cache, v_cache, head_dim)) {
+    if (attention_decode_fits(q, k_cache, v_cache, head_dim)) {
         decode_attention(dst, q, k_cache, v_cache, kv_len, head_dim, n_heads, n_kv_heads);
         return;
     }

@@ -1,0 +1,99 @@
+"""Decode attention at the edges of its ranges: one workgroup's one or two
+passes, the switch to several ranges, ranges of uneven length, up to 8, 16 and
+more ranges per head, heads of 16 and 32 lanes; and a decode step's rotation
+inside it.
+
+Bar: float64 numpy, 2e-6 normwise: a score is a 128-term fp32 sum (relative
+error about sqrt(128) 2^-24 of |q||k| / sqrt(hd), about 7e-7 in the exponent
+for N(0,1) rows), and the weighted sum adds as much.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from oracle.oracle import normwise_err
+from test_gpu_attention import down, up, want_attention
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(128, 32, 32, 63), (128, 32, 32, 129), (128, 32, 8, 256), (128, 32, 32, 257), (128, 32, 32, 513),
+         (128, 32, 8, 1025), (128, 32, 32, 2048), (128, 8, 2, 1153), (128, 1, 1, 9001), (128, 5, 5, 3333),
+         (64, 32, 8, 512), (64, 32, 8, 513), (64, 8, 4, 2805), (96, 12, 4, 700), (16, 4, 2, 2049), (4, 2, 1, 8193),
+         (128, 300, 100, 400)]
+
+
+@pytest.mark.parametrize("hd,nh,nkv,kv_len", CASES)
+def test_decode_ranges(holo, synth, hd, nh, nkv, kv_len):
+    print(f"case decode ranges hd {hd} heads {nh}/{nkv} kv_len {kv_len}", flush=True)
+    lib = holo.lib()
+    kv_dim = nkv * hd
+    q, kc, vc = (synth.normal(n, seed=40 + i) for i, n in enumerate((nh * hd, kv_len * kv_dim, kv_len * kv_dim)))
+    kc[-kv_dim:] *= 3.0  # the last position carries weight
+    dq, dk, dv = up(holo, q), up(holo, kc), up(holo, vc)
+    outs = []
+    for _ in range(2):
+        d = up(holo, np.full(nh * hd + 8, 7.0, np.float32))
+        lib.cuda_multi_head_attention(d.ptr, dq.ptr, dk.ptr, dv.ptr, kv_len, hd, nh, nkv)
+        lib.cuda_sync()
+        outs.append(down(d, nh * hd + 8))
+    holo.check("decode ranges")
+    assert np.array_equal(outs[0], outs[1])
+    assert np.all(outs[0][nh * hd:] == 7.0)
+    K, V = (a.reshape(kv_len, nkv, hd).astype(np.float64) for a in (kc, vc))
+    assert normwise_err(outs[0][:nh * hd], want_attention(q, K, V, nh, nkv, hd, kv_len)) <= 2e-6
+
+
+@pytest.mark.parametrize("hd,nh,nkv,pos", [(128, 4, 4, 0), (128, 8, 2, 255), (128, 8, 2, 700), (64, 4, 2, 1300),
+                                           (32, 4, 1, 40)])
+def test_decode_step_rotation(holo, synth, hd, nh, nkv, pos):
+    """One layer, one token, through holo_llama_forward: the key row it leaves
+    in the cache is the rotated product (cuda_rope_apply on holo_matmul's key
+    and query), its neighbours are untouched, and the logits are those of the
+    same layer run op by op."""
+    lib = holo.lib()
+    dim, kv_dim, ffn, vocab, max_seq = nh * hd, nkv * hd, 256, 64, pos + 3
+    F32 = 0
+    shapes = {"wq": (dim, dim), "wk": (kv_dim, dim), "wv": (kv_dim, dim), "wo": (dim, dim), "w1": (ffn, dim),
+              "w2": (dim, ffn), "w3": (ffn, dim)}
+    W = {n: up(holo, synth.normal(o * i, seed=60 + k) / np.float32(np.sqrt(i))) for k, (n, (o, i)) in enumerate(shapes.items())}
+    emb, head = up(holo, synth.normal(vocab * dim, seed=70)), up(holo, synth.normal(vocab * dim, seed=71) / np.float32(np.sqrt(dim)))
+    k0, v0 = synth.normal(max_seq * kv_dim, seed=72), synth.normal(max_seq * kv_dim, seed=73)
+    dk, dv, logits = up(holo, k0), up(holo, v0), holo.DeviceBuffer(4 * vocab)
+    layer = (holo.LlamaLayer * 1)()
+    for n in shapes:
+        setattr(layer[0], n, W[n].ptr)
+        setattr(layer[0], n + "_type", F32)
+    m = holo.LlamaModel(n_layers=1, dim=dim, n_heads=nh, n_kv_heads=nkv, head_dim=hd, ffn_dim=ffn, vocab=vocab,
+                        max_seq=max_seq, rms_eps=1e-5, rope_base=10000.0, tok_emb=emb.ptr, emb_type=F32,
+                        output=head.ptr, out_type=F32, key_cache=dk.ptr, value_cache=dv.ptr, layers=layer)
+    tok = (C.c_int * 1)(17)
+    assert lib.holo_llama_forward(C.byref(m), tok, 1, pos, logits.ptr, 0) == 0
+    lib.cuda_sync()
+    holo.check("decode step")
+    # op by op (no norms in this model)
+    x, q, k, v, att, t = (holo.DeviceBuffer(4 * n) for n in (dim, dim, kv_dim, kv_dim, dim, dim))
+    h1, h3, want = holo.DeviceBuffer(4 * ffn), holo.DeviceBuffer(4 * ffn), holo.DeviceBuffer(4 * vocab)
+    lib.cuda_get_embedding_f32(x.ptr, emb.ptr, 17, dim, vocab)
+    for d, n in ((q, "wq"), (k, "wk"), (v, "wv")):
+        lib.holo_matmul(d.ptr, W[n].ptr, x.ptr, *shapes[n], F32)
+    lib.cuda_rope_apply(q.ptr, k.ptr, pos, hd, nh, nkv, 10000.0)
+    kw, vw = k0.copy(), v0.copy()
+    kw[pos * kv_dim:(pos + 1) * kv_dim], vw[pos * kv_dim:(pos + 1) * kv_dim] = down(k, kv_dim), down(v, kv_dim)
+    gk, gv = down(dk, max_seq * kv_dim), down(dv, max_seq * kv_dim)
+    assert np.array_equal(gv, vw)
+    assert np.array_equal(np.delete(gk.reshape(max_seq, -1), pos, 0), np.delete(kw.reshape(max_seq, -1), pos, 0))
+    assert normwise_err(gk, kw) <= 2e-7  # one rounding per rotated value
+    ck, cv = up(holo, kw), up(holo, vw)
+    lib.cuda_multi_head_attention(att.ptr, q.ptr, ck.ptr, cv.ptr, pos + 1, hd, nh, nkv)
+    lib.holo_matmul(t.ptr, W["wo"].ptr, att.ptr, dim, dim, F32)
+    lib.cuda_vec_add(x.ptr, x.ptr, t.ptr, dim)
+    lib.holo_matmul(h1.ptr, W["w1"].ptr, x.ptr, ffn, dim, F32)
+    lib.holo_matmul(h3.ptr, W["w3"].ptr, x.ptr, ffn, dim, F32)
+    lib.cuda_silu_mul(h1.ptr, h1.ptr, h3.ptr, ffn)
+    lib.holo_matmul(t.ptr, W["w2"].ptr, h1.ptr, dim, ffn, F32)
+    lib.cuda_vec_add(x.ptr, x.ptr, t.ptr, dim)
+    lib.holo_matmul(want.ptr, head.ptr, x.ptr, vocab, dim, F32)
+    lib.cuda_sync()
+    holo.check("op by op")
+    assert normwise_err(down(logits, vocab), down(want, vocab)) <= 5e-6
