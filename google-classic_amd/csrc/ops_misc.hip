@@ -254,22 +254,24 @@ __device__ __forceinline__ void split8_f16(const float x[8], af16x8 &hi, af16x8 
     }
 }
 
-template <int HD>
-__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const float *q, const float *kc,
+// NW waves per workgroup: 4 (two workgroups per CU) or, where there are too
+// few workgroups for that, 8 (one per CU).
+template <int HD, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_mfma_k(float *out, const float *q, const float *kc,
                                                            const float *vc, int rows, int pos0, int n_heads,
                                                            int n_kv_heads, int nqb)
 {
     constexpr int NQ = HD / 16;  // 16-dim chunks of a row: the K of one f16 score MFMA
     constexpr int VB = HD / 32;  // output blocks: lane i covers dims VB*i .. VB*i + VB - 1
     extern __shared__ float amf_lds[];
-    // the waves' outputs [4 waves][32 queries][HD + 1]: the merge pass reads
+    // the waves' outputs [NW waves][32 queries][HD + 1]: the merge pass reads
     // consecutive dims of a query row (one bank each), the stores from the
     // MFMA layout put the 32 queries of a register on distinct banks
     constexpr int OS = HD + 1;
     float *lo = amf_lds;
-    float *lm = lo + 4 * 32 * OS;              // [4][32] running max per query
-    float *ll = lm + 4 * 32;                   // [4][64] running sum per lane
-    float *lw = ll + 4 * 64;                   // [4][32] merge weight of each wave per query
+    float *lm = lo + NW * 32 * OS;             // [NW][32] running max per query
+    float *ll = lm + NW * 32;                  // [NW][64] running sum per lane
+    float *lw = ll + NW * 64;                  // [NW][32] merge weight of each wave per query
     // (head, query block) of this workgroup. Query blocks go out by rank k:
     // the first ceil(nqb/2) ranks heaviest first, the rest lightest first, so
     // ranks k and k + ceil(nqb/2), which share CUs as the second workgroup
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
     // loop.
     constexpr int QS = HD + 8;
     _Float16 *qh = (_Float16 *)amf_lds, *ql = qh + 32 * QS;
-    for (int e = threadIdx.x; e < 32 * (HD / 4); e += 256) {
+    for (int e = threadIdx.x; e < 32 * (HD / 4); e += 64 * NW) {
         const int r = e / (HD / 4), c4 = e - r * (HD / 4);
         const float4 x = *(const float4 *)(q + (int64_t)min(q0 + r, rows - 1) * q_dim + (int64_t)h * HD + 4 * c4);
         _Float16 hv[4], lv[4];
@@ -324,14 +326,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
     // zeros (their scores are masked and their probabilities 0)
     const float *khead = kc + (int64_t)kvh * HD, *vhead = vc + (int64_t)kvh * HD;
     const uint32_t rowb = (uint32_t)kv_dim * 4u;
-    const uint32_t kvo = (uint32_t)j * rowb + 32u * (uint32_t)hh;          // key j, dims 8hh ..
+    // Keys come DH dims of whole rows at a time, LR lanes a row, and reach
+    // their lanes through the wave's LDS stage (rows padded by 16 bytes: the
+    // operand reads of 16 rows take 64 distinct banks).  Loaded straight to
+    // its lane, 16 bytes of 32 rows an instruction, a tile's keys took the
+    // CU's address unit about 1,000 cycles of 1,800 a tile, here 300 (192 rows
+    // at 1000, 32 heads on 8: 29.3 -> 22.7 us, 500 at 3000, 8 heads: 69 -> 49,
+    // 512 at 0, 32 heads: 21.0 -> 17.8).
+    constexpr int DH = HD < 64 ? HD : 64, LR = DH / 4, RPI = 64 / LR, NI = 32 / RPI, KS = DH + 4;
+    float *kst = (float *)(ql + 32 * QS) + wave * (32 * KS);
+    const uint32_t kvo = (uint32_t)(lane / LR) * rowb + 16u * (uint32_t)(lane % LR);
+    float *const kput = kst + (lane / LR) * KS + 4 * (lane % LR);
+    const float *const kget = kst + j * KS + 8 * hh;
     const uint32_t vvo = 4u * (uint32_t)hh * rowb + 4u * VB * (uint32_t)j;  // key 4hh + .., dims VB j ..
     float m = -INFINITY, l = 0.f;
     v16f o[VB];
 #pragma unroll
     for (int b = 0; b < VB; b++) o[b] = v16f{};
 
-    for (int t = wave; t < ntiles; t += 4) {
+    for (int t = wave; t < ntiles; t += NW) {
         const int key0 = t * 32;
         // Sᵀ = K Qᵀ on v_mfma_f32_32x32x16_f16 with both operands split:
         // lane j + 32hh supplies dims 16c + 8hh .. 16c + 8hh + 7 of key j (A) and
@@ -342,13 +355,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
             (void *)(khead + (int64_t)key0 * kv_dim), (short)0, (int)((uint32_t)nk * rowb), kRawBufWord3);
         const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(vhead + (int64_t)key0 * kv_dim), (short)0, (int)((uint32_t)nk * rowb), kRawBufWord3);
-        float4 kr[2 * NQ];
+        float4 kr[HD / DH][NI];
 #pragma unroll
-        for (int c = 0; c < NQ; c++) {
-            kr[2 * c] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)(kvo + 64 * c), 0, 0));
-            kr[2 * c + 1] =
-                __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)(kvo + 64 * c + 16), 0, 0));
-        }
+        for (int f = 0; f < HD / DH; f++)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+                kr[f][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                          rk, (int)(kvo + 4 * DH * f), (int)((uint32_t)(RPI * i) * rowb), 0));
         // the output product's 16 key row pieces, loaded with the keys so that
         // their round trip runs under the scores
         float vv[16][VB];
@@ -372,8 +385,15 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
         v16f s = v16f{};
 #pragma unroll
         for (int c = 0; c < NQ; c++) {
-            const float kv[8] = {kr[2 * c].x,     kr[2 * c].y,     kr[2 * c].z,     kr[2 * c].w,
-                                 kr[2 * c + 1].x, kr[2 * c + 1].y, kr[2 * c + 1].z, kr[2 * c + 1].w};
+            if (c % (DH / 16) == 0) {
+                // this wave's own stage: its LDS accesses stay in order, so the
+                // reads below need no barrier, nor these writes after the last ones
+#pragma unroll
+                for (int i = 0; i < NI; i++) *(float4 *)(kput + RPI * i * KS) = kr[c / (DH / 16)][i];
+            }
+            const float4 ka = *(const float4 *)(kget + 16 * (c % (DH / 16)));
+            const float4 kb = *(const float4 *)(kget + 16 * (c % (DH / 16)) + 4);
+            const float kv[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
             af16x8 kh, kl;
             split8_f16(kv, kh, kl);
             const af16x8 bh = *(const af16x8 *)(qhr + 16 * c), bl = *(const af16x8 *)(qlr + 16 * c);
@@ -426,7 +446,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
         }
     }
 
-    // merge the 4 waves: O = sum_w 2^(m_w - M) O_w / L, L = sum_w 2^(m_w - M) l_w
+    // merge the waves: O = sum_w 2^(m_w - M) O_w / L, L = sum_w 2^(m_w - M) l_w
     __syncthreads();  // every wave is done with the query rows in lo
 #pragma unroll
     for (int b = 0; b < VB; b++)
@@ -438,49 +458,64 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_k(float *out, const 
     if (hh == 0) lm[wave * 32 + j] = m;
     ll[wave * 64 + lane] = l;
     __syncthreads();
-    // each query's four weights 2^(m_w - M) / L, once per query rather than
+    // each query's weights 2^(m_w - M) / L, once per query rather than
     // per output element
     if (threadIdx.x < 32) {
         const int qj = threadIdx.x;
         float M = lm[qj];
 #pragma unroll
-        for (int w = 1; w < 4; w++) M = fmaxf(M, lm[w * 32 + qj]);
-        float wg[4], L = 0.f;
+        for (int w = 1; w < NW; w++) M = fmaxf(M, lm[w * 32 + qj]);
+        float wg[NW], L = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
+        for (int w = 0; w < NW; w++) {
             const float mw = lm[w * 32 + qj];
             wg[w] = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
             L += wg[w] * (ll[w * 64 + qj] + ll[w * 64 + 32 + qj]);
         }
 #pragma unroll
-        for (int w = 0; w < 4; w++) lw[w * 32 + qj] = wg[w] / L;
+        for (int w = 0; w < NW; w++) lw[w * 32 + qj] = wg[w] / L;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < 32 * HD; e += 256) {
+    for (int e = threadIdx.x; e < 32 * HD; e += 64 * NW) {
         const int qj = e / HD, d = e - qj * HD;  // consecutive threads: consecutive dims of one row
         if (q0 + qj >= rows) continue;
         float O = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) O += lw[w * 32 + qj] * lo[(w * 32 + qj) * OS + d];
+        for (int w = 0; w < NW; w++) O += lw[w * 32 + qj] * lo[(w * 32 + qj) * OS + d];
         out[(int64_t)(q0 + qj) * q_dim + (int64_t)h * HD + d] = O;
     }
+}
+
+template <int HD, int NW>
+static void launch_attn_prefill_waves(float *out, const float *q, const float *kc, const float *vc, int rows, int pos0,
+                                      int n_heads, int n_kv_heads)
+{
+    constexpr size_t merge = (size_t)(NW * 32 * (HD + 1) + NW * 32 + NW * 64 + NW * 32) * sizeof(float);
+    constexpr size_t loop = (size_t)2 * 32 * (HD + 8) * 2 + (size_t)NW * 32 * ((HD < 64 ? HD : 64) + 4) * sizeof(float);
+    constexpr size_t lds = merge > loop ? merge : loop;
+    static bool attr = false;
+    if (!attr) {
+        HOLO_CHECK(hipFuncSetAttribute((const void *)attn_prefill_mfma_k<HD, NW>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr = true;
+    }
+    const int nqb = (rows + 31) / 32;
+    hipLaunchKernelGGL((attn_prefill_mfma_k<HD, NW>), dim3((unsigned)(nqb * n_heads)), dim3(64 * NW), lds, stream(),
+                       out, q, kc, vc, rows, pos0, n_heads, n_kv_heads, nqb);
+    HOLO_LAUNCH_CHECK();
 }
 
 template <int HD>
 static void launch_attn_prefill_mfma(float *out, const float *q, const float *kc, const float *vc, int rows, int pos0,
                                      int n_heads, int n_kv_heads)
 {
-    constexpr size_t lds = (size_t)(4 * 32 * (HD + 1) + 4 * 32 + 4 * 64 + 4 * 32) * sizeof(float);
-    static bool attr = false;
-    if (!attr) {
-        HOLO_CHECK(hipFuncSetAttribute((const void *)attn_prefill_mfma_k<HD>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr = true;
-    }
-    const int nqb = (rows + 31) / 32;
-    hipLaunchKernelGGL(attn_prefill_mfma_k<HD>, dim3((unsigned)(nqb * n_heads)), dim3(256), lds, stream(), out, q, kc,
-                       vc, rows, pos0, n_heads, n_kv_heads, nqb);
-    HOLO_LAUNCH_CHECK();
+    // eight waves where four leave a CU one wave per SIMD and there are tiles
+    // for them: 192 rows at 1000, 32 heads: 30.0 -> 29.3 us before the keys
+    // were staged; with more workgroups two of four waves share a CU and the
+    // shorter merge is the better one
+    const bool wide = (rows + 31) / 32 * n_heads <= num_cus() && pos0 + rows > 4 * 32;
+    if (wide) launch_attn_prefill_waves<HD, 8>(out, q, kc, vc, rows, pos0, n_heads, n_kv_heads);
+    else launch_attn_prefill_waves<HD, 4>(out, q, kc, vc, rows, pos0, n_heads, n_kv_heads);
 }
 
 // ---- Q6_K GEMV (cuda_matmul_q6_k) ---------------------------------------------------
