@@ -79,9 +79,10 @@ constexpr int kFrWaves = 8;
 // 11; three rows 13.7 against 11.4.
 constexpr int kFrMinRows = 3;
 // From 64 rows the estimates choose between this and the 64 x 256 tiles (us
-// there against here: 256 x 4096 x 4096 46.0 / 33.7, 192 x 11008 x 4096 73.7 /
-// 62.4, 512 x 1024 x 4096 44.9 / 27.0, 256 x 11008 x 4096 73.2 / 77.2), and
-// the tiles run where they fill every CU twice (512 x 4096 x 4096: level) or
+// there against here: 256 x 4096 x 4096 45.7 / 32.2, 192 x 11008 x 4096 71.4 /
+// 59.5, 512 x 1024 x 4096 44.7 / 26.5, 256 x 11008 x 4096 72.8 / 74.2), and
+// the tiles run where they fill every CU twice (512 x 4096 x 4096: 65.5 / 55.0,
+// 916 x 4082 x 2336 Q8_0: 74.7 / 119.8) or
 // this would take more than three rounds of workgroups (764 x 14319 x 1792
 // Q6_K, eleven rounds: 128 / 202: the weights leave the caches between the
 // row tiles), and above this many rows.
@@ -674,20 +675,24 @@ struct FrPlan {
 };
 
 // Picks the plan with the least estimated time, fitted to a sweep of mt, ct
-// and ks over 4096 x 4096, 11008 x 4096 and 4096 x 11008 at 2 to 192 rows.
-// Per unit of a workgroup's longest wave, in us: the load unit takes 0.16 per
-// column tile and 0.93 per row tile (every wave reads its own activations),
-// the vector unit 0.34 per column tile to unpack and 0.13 per product tile.
-// A round of workgroups over the CUs adds 2.8 (first loads, sums, stores), a
-// second part of K its exchange, 2.5.  At 16 rows of 11008 x 4096: 48 columns
-// and one round 16.2, 32 columns 18.3, 64 columns 19.0, 16 columns 19.3.
+// and ks over 30 shapes of all types, 16 to 400 rows, out 500 to 14336, in
+// 1024 to 14336 (the picks there are within 3% of the best plan).  In us: per
+// unit of a workgroup's longest wave 0.75 per row tile (every wave reads its
+// own activations), 0.73 per column tile (its loads and unpacking) and 0.32
+// per product tile; a round of workgroups over the CUs 0.75, a second part of
+// K its exchange, 3.2; and at least the activation operands of all workgroups
+// out of L2, 22.5 TB/s.  Above 32 rows 64-row tiles: more, narrower row tiles
+// read the weights again (64 x 11008 x 4096: 26.4 against 32.8).  At 16 rows
+// of 11008 x 4096: 48 columns and one round 16.0, 32 columns 18.3, 64 columns
+// 18.9, 16 columns 19.2.
 FrPlan few_plan(int kind, const int *N, int nmat, int M, int nb)
 {
     FrPlan best = {};
     const int nu = (nb + 7) / 8;
-    const float type = kind == EW_Q8_0 ? 1.35f : kind == EW_Q6_K ? 1.3f : kind == EW_Q4_K ? 1.1f : 1.f;
+    const float type = kind == EW_Q8_0 ? 1.15f : kind == EW_Q6_K ? 1.39f : kind == EW_Q4_K ? 1.09f : 1.f;
     for (int mt = 1; mt <= 4; mt *= 2) {
         if (mt > 1 && 16 * mt >= 2 * M) break;
+        if (mt < 4 && M > 32) continue;
         for (int ct = 1; ct <= (kind == EW_Q8_0 && mt == 4 ? 3 : 4); ct++) {  // 64 x 64 Q8_0 spills
             int nct = 0;
             for (int i = 0; i < nmat; i++) nct += (N[i] + 16 * ct - 1) / (16 * ct);
@@ -698,10 +703,9 @@ FrPlan few_plan(int kind, const int *N, int nmat, int M, int nb)
                     break;
                 const int units = (nu + kFrWaves * ks - 1) / (kFrWaves * ks);
                 const int rounds = (nct * nrt * ks + num_cus() - 1) / num_cus();
-                float us = (float)rounds * (2.8f + type * (float)units * (0.5f * ct + 0.93f * mt + 0.13f * ct * mt)) +
-                                 (ks > 1 ? 2.5f : 0.f);
-                // the activation operands of all workgroups out of L2, 12 TB/s
-                us = std::max(us, (float)((int64_t)nct * ((M + 15) / 16) * nb * 2048) * (1.f / 12e6f));
+                float us = (float)rounds * (0.75f + type * (float)units * (0.73f * ct + 0.75f * mt + 0.32f * ct * mt)) +
+                           (ks > 1 ? 3.2f : 0.f);
+                us = std::max(us, (float)((int64_t)nct * ((M + 15) / 16) * nb * 2048) * (1.f / 22.5e6f));
                 if (best.mt == 0 || us < best.us) best = {mt, ct, ks, nct, nrt, rounds, us};
             }
         }
@@ -871,7 +875,7 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     int nl = 0, counters = 0;
     size_t parts = 0;
     bool many = false;
-    float here = 5.7f, tiled = 0.f;  // estimates, us (5.7: the split and two launches)
+    float here = 7.6f, tiled = 0.f;  // estimates, us (7.6: the split and two launches)
     bool done[kExactMats] = {false, false, false};
     for (int i = 0; i < nmat; i++) {
         if (done[i]) continue;
@@ -903,7 +907,11 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
             counters = std::max(counters, l.p.nct * l.p.nrt);
         }
     }
-    if (M >= 64 && (many || tiled <= 1.1f * here)) return false;
+    // From 64 rows on, the other tiling where it is estimated 6% better (both
+    // sides measured on 70 shapes: the taken one is the faster or within 5% for
+    // all that are not `full`): 192 x 11008 x 4096 Q4_0 here 59.5 us, there 71.4;
+    // 231 x 6825 x 5632 Q6_K 92.3 and 87.1; 1015 x 890 x 4864 Q8_0 71.2 and 59.4.
+    if (M >= 64 && (many || tiled <= 0.94f * here)) return false;
     const int ntm = (M + 15) / 16;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t ob = up((size_t)ntm * nb * 2048), sb = need_sx ? up((size_t)ntm * nb * 64) : 0, rb = up((size_t)M * 4),
