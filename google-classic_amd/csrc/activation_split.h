@@ -27,16 +27,23 @@ namespace holo {
 // [rows / 16][block][16]; n_zero counters at `zero` are cleared.  There the
 // low half of an infinite value is zero, so that the products of a row with
 // infinities are the infinities (and NaNs) that fp32 gives.
+// PART (with OPS): gridDim.y workgroups share a row: each finds the row's
+// scale from all of it and splits and stores float4s part * blockIdx.y ..
+// of it (part a multiple of 8 and at most NT), which it loads a second time.
+// The row's largest |silu(g) u| comes from the hardware's exp2 and reciprocal
+// (off by |g| 2^-23 and a few ulp: under 2^-16 up to |g| = 88, where silu ends);
+// where that could change the power of two, it is found again with expf.
 namespace {
 enum XSplitMode { XS_PLAIN = 0, XS_SWIGLU = 1, XS_NORM = 2 };
 
-template <int NV, int MODE, int NT = 256, bool OPS = false>
+template <int NV, int MODE, int NT = 256, bool OPS = false, bool PART = false>
 __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2 *__restrict__ Al,
                                                     float *__restrict__ Sx, float *__restrict__ Rs,
                                                     const float *__restrict__ X, const float *__restrict__ U,
                                                     const float *__restrict__ NW, int K, float eps, uint32_t *zero,
-                                                    int n_zero)
+                                                    int n_zero, int part)
 {
+    static_assert(OPS || !PART);
     __shared__ float red[16];
     const int n4 = K >> 2;
     const int64_t r4 = (int64_t)blockIdx.x * n4;
@@ -59,10 +66,25 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         if constexpr (MODE == XS_NORM)
             wv[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
     }
+    // PART: this thread's own float4 (past its part: none, zeros)
+    const int pi = PART ? (int)(blockIdx.y * part + threadIdx.x) : 0;
+    const bool mine = (int)threadIdx.x < part && pi < n4;
+    float4 pv, pw;
+    if constexpr (PART) {
+        const int o = mine ? pi * 16 : K * 4;
+        pv = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
+        if constexpr (MODE == XS_SWIGLU)
+            pw = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
+        if constexpr (MODE == XS_NORM)
+            pw = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
+    }
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-        if constexpr (MODE == XS_SWIGLU) {
+        if constexpr (MODE == XS_SWIGLU && PART) {
+            auto sg = [](float g) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504f)); };
+            v[j] = make_float4(sg(v[j].x) * wv[j].x, sg(v[j].y) * wv[j].y, sg(v[j].z) * wv[j].z, sg(v[j].w) * wv[j].w);
+        } else if constexpr (MODE == XS_SWIGLU) {
             const float4 u = wv[j];
             v[j].x = (v[j].x / (1.0f + expf(-v[j].x))) * u.x;
             v[j].y = (v[j].y / (1.0f + expf(-v[j].y))) * u.y;
@@ -88,6 +110,20 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         am = fmaxf(am, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
     }
     am = block_reduce<true>(am, red);
+    if constexpr (MODE == XS_SWIGLU && PART) {
+        // within 2^-15 of a power of two, tiny (the reciprocal flushes), or not finite
+        if (((__float_as_uint(am) + 256u) & 0x7FFFFFu) < 512u || am < 1e-30f) {
+            am = 0.f;
+            for (int j = 0; j < NV; j++) {
+                const int o = (int)(threadIdx.x + NT * j) * 16;
+                const float4 g = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
+                const float4 u = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
+                am = fmaxf(am, fmaxf(fmaxf(fabsf((g.x / (1.0f + expf(-g.x))) * u.x), fabsf((g.y / (1.0f + expf(-g.y))) * u.y)),
+                                     fmaxf(fabsf((g.z / (1.0f + expf(-g.z))) * u.z), fabsf((g.w / (1.0f + expf(-g.w))) * u.w))));
+            }
+            am = block_reduce<true>(am, red);
+        }
+    }
     // 2^e with a * 2^e in [2^14, 2^15); e = 0 for a zero or non-finite row
     int e = 0;
     if (am > 0.f && am <= 3.4028235e38f) {
@@ -95,14 +131,25 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         (void)frexpf(am, &ea);  // am = f * 2^ea, f in [0.5, 1)
         e = 15 - ea;
     }
-    if (threadIdx.x == 0) Rs[blockIdx.x] = ldexpf(1.0f, -e);
-    if (OPS && blockIdx.x == 0)
+    if (threadIdx.x == 0 && (!PART || blockIdx.y == 0)) Rs[blockIdx.x] = ldexpf(1.0f, -e);
+    if (OPS && blockIdx.x == 0 && (!PART || blockIdx.y == 0))
         for (int j = threadIdx.x; j < n_zero; j += NT) zero[j] = 0;
+    if constexpr (PART) {
+        if constexpr (MODE == XS_SWIGLU) {
+            pv.x = (pv.x / (1.0f + expf(-pv.x))) * pw.x;
+            pv.y = (pv.y / (1.0f + expf(-pv.y))) * pw.y;
+            pv.z = (pv.z / (1.0f + expf(-pv.z))) * pw.z;
+            pv.w = (pv.w / (1.0f + expf(-pv.w))) * pw.w;
+        }
+        if constexpr (MODE == XS_NORM)
+            pv = make_float4(pv.x * scale * pw.x, pv.y * scale * pw.y, pv.z * scale * pw.z, pv.w * scale * pw.w);
+    }
 #pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int i = threadIdx.x + NT * j;
-        if (NT * j >= n4) break;  // uniform: no lane of this or a later j is live
-        const float y[4] = {ldexpf(v[j].x, e), ldexpf(v[j].y, e), ldexpf(v[j].z, e), ldexpf(v[j].w, e)};
+    for (int j = 0; j < (PART ? 1 : NV); j++) {
+        const int i = PART ? pi : (int)threadIdx.x + NT * j;
+        const float4 x = PART ? pv : v[j];
+        if (!PART && NT * j >= n4) break;  // uniform: no lane of this or a later j is live
+        const float y[4] = {ldexpf(x.x, e), ldexpf(x.y, e), ldexpf(x.z, e), ldexpf(x.w, e)};
         _Float16 h[4], l[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -117,13 +164,17 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         s += __shfl_xor(s, 4, 64);
         if constexpr (OPS) {
             // float4 i is block i / 8, weights 4 (i % 8) .. of it: operand lane
-            // row + 16 (i % 4), half (i % 8) / 4 of its 16 bytes, order 0, 2, 1, 3
-            if (i < n4) {
+            // row + 16 (i % 4), half (i % 8) / 4 of its 16 bytes, order 0, 2, 1, 3.
+            // Lanes i and i + 4 trade halves: one stores the high operand's 16
+            // bytes, the other the low one's.
+            const bool up = (i >> 2) & 1;
+            const uint32_t h0 = __builtin_bit_cast(uint32_t, h2{h[0], h[2]}), h1 = __builtin_bit_cast(uint32_t, h2{h[1], h[3]});
+            const uint32_t l0 = __builtin_bit_cast(uint32_t, h2{l[0], l[2]}), l1 = __builtin_bit_cast(uint32_t, h2{l[1], l[3]});
+            const uint32_t t0 = (uint32_t)__shfl_xor((int)(up ? h0 : l0), 4, 64), t1 = (uint32_t)__shfl_xor((int)(up ? h1 : l1), 4, 64);
+            if (PART ? mine : i < n4) {
                 const int64_t b = (int64_t)(blockIdx.x >> 4) * (n4 >> 3) + (i >> 3);
                 const int m = blockIdx.x & 15;
-                const int64_t o = ((b * 128 + m + 16 * (i & 3)) << 1) + ((i >> 2) & 1);
-                Ah[o] = make_uint2(__builtin_bit_cast(uint32_t, h2{h[0], h[2]}), __builtin_bit_cast(uint32_t, h2{h[1], h[3]}));
-                Ah[o + 128] = make_uint2(__builtin_bit_cast(uint32_t, h2{l[0], l[2]}), __builtin_bit_cast(uint32_t, h2{l[1], l[3]}));
+                ((uint4 *)Ah)[b * 128 + m + 16 * (i & 3) + (up ? 64 : 0)] = up ? make_uint4(t0, t1, l0, l1) : make_uint4(h0, h1, t0, t1);
                 if (Sx && (i & 7) == 0) Sx[b * 16 + m] = s;
             }
         } else if (i < n4) {

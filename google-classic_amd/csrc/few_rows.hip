@@ -34,7 +34,7 @@
 // unit, three quarters busy, mostly with activation operands (4 bytes per
 // value, read once per workgroup), then the unpacking.  Measured with the
 // split launch, us, one GEMV per row -> this kernel (Q4_0, 16 rows):
-// 4096 x 4096 70.5 -> 11.9, 11008 x 4096 118.6 -> 15.9, 4096 x 11008 121.4 ->
+// 4096 x 4096 70.5 -> 11.9, 11008 x 4096 118.6 -> 14.9, 4096 x 11008 121.4 ->
 // 20.2; 64 rows, 64 x 256 tiles -> this kernel: 39.0 -> 16.1, 40.3 -> 24.9,
 // 73.2 -> 31.2.
 #include "common.h"
@@ -931,14 +931,32 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     uint8_t *A = ws;
     float *Sx = need_sx ? (float *)(ws + ob) : nullptr, *Rs = (float *)(ws + ob + sb);
     uint32_t *cnt = (uint32_t *)(ws + ob + sb + rb);
+    // Few rows leave most CUs idle: four workgroups a row (each of at most
+    // `most` float4s) while they fit the CUs.  23 rows, alone -> four -> eight:
+    // SwiGLU 11008 wide 8.6 -> 6.6 -> 7.5 us, the norm 4096 wide 5.0 -> 4.6 ->
+    // 4.5, plain 4.9 -> 4.4 -> 4.3.
+    int shares = 1, part = 0;
+    auto share = [&](int most) {
+        const int n4 = K >> 2, need = (n4 + most - 1) / most;
+        shares = std::max(need, std::min(4, num_cus() / M));
+        if (shares * M > num_cus()) shares = 1;
+        part = ((n4 + shares - 1) / shares + 7) & ~7;
+        return shares > 1;
+    };
     auto split = [&](auto kern, int nt) {
-        hipLaunchKernelGGL(kern, dim3(M), dim3(nt), 0, stream(), (uint2 *)A, (uint2 *)nullptr, Sx, Rs, X, U, NW, K, eps,
-                           cnt, counters);
+        hipLaunchKernelGGL(kern, dim3(M, shares), dim3(nt), 0, stream(), (uint2 *)A, (uint2 *)nullptr, Sx, Rs, X, U, NW, K,
+                           eps, cnt, counters, part);
     };
     const bool small = K <= 4096;
     // the normed form keeps rms_norm_rows4_k's 256 threads and summation order
-    if (NW) small ? split(xsplit_row_k<4, XS_NORM, 256, true>, 256) : split(xsplit_row_k<16, XS_NORM, 256, true>, 256);
+    if (NW && share(256))
+        small ? split(xsplit_row_k<4, XS_NORM, 256, true, true>, 256) : split(xsplit_row_k<16, XS_NORM, 256, true, true>, 256);
+    else if (NW) small ? split(xsplit_row_k<4, XS_NORM, 256, true>, 256) : split(xsplit_row_k<16, XS_NORM, 256, true>, 256);
+    else if (U && share(1024))
+        small ? split(xsplit_row_k<1, XS_SWIGLU, 1024, true, true>, 1024) : split(xsplit_row_k<4, XS_SWIGLU, 1024, true, true>, 1024);
     else if (U) small ? split(xsplit_row_k<1, XS_SWIGLU, 1024, true>, 1024) : split(xsplit_row_k<4, XS_SWIGLU, 1024, true>, 1024);
+    else if (share(1024))
+        small ? split(xsplit_row_k<1, XS_PLAIN, 1024, true, true>, 1024) : split(xsplit_row_k<4, XS_PLAIN, 1024, true, true>, 1024);
     else small ? split(xsplit_row_k<1, XS_PLAIN, 1024, true>, 1024) : split(xsplit_row_k<4, XS_PLAIN, 1024, true>, 1024);
     HOLO_LAUNCH_CHECK();
     for (int i = 0; i < nl; i++) {
