@@ -624,6 +624,201 @@ __global__ __launch_bounds__(256) void gemv_q6_k2_k(float *dst, const uint8_t *M
     }
 }
 
+// Many rows: the same tasks with everything through LDS.  A wave's pass reads
+// 16 superblocks of a row (3360 contiguous bytes) in whole 16-byte pieces, puts
+// them into its own stage and takes its tasks' runs from there.  Loaded
+// straight to its lane (gemv_q6_k2_k), a task's runs and activations are a
+// dozen loads of 64 scattered pieces, and the CU's address unit takes a cycle
+// for nearly every piece.  A wave walks row groups, kQ6Rows at a time, the next
+// pass's pieces in flight.
+//
+// Activations: 24-bit fixed point per group of 16 (the weights' scale groups),
+// xi = rint(x * 127 * 65536 / amax) = 65536 h + 256 m + l with int8 h, m, l, and
+// the integer dots with q - 32 (the offset through -32 times the planes' sums)
+// on v_dot4: exact up to a group's one rounding (10.1 -> 7.8 M vector
+// instructions).  32000 x 4096, us, three matrices in turn: straight loads
+// 30.3, staged 27.7, with integer dots 26.0; one matrix repeated 28.6 -> 23.6
+// (its 107.7 MB take 21.4 at a copy's rate); against float64 1.2e-7 normwise,
+// fp32 products 1.7e-7.  What is left: the first loads, the conversion (2 of 7.8 M
+// vector instructions) and the last rows.
+constexpr int kQ6Waves = 8, kQ6Rows = 2;
+constexpr int kQ6Run = 16 * 210;                          // bytes of a row in a pass
+constexpr int kQ6Pieces = (kQ6Run + 14 + 15) / 16;        // with the start rounded down to 16
+constexpr int kQ6Loads = (kQ6Pieces + 63) / 64;
+constexpr int kQ6Stage = 16 * kQ6Pieces + 16;             // a run's window reads up to 4 bytes past it
+
+// DPP quad permutation.
+template <int CTRL>
+__device__ __forceinline__ float q6_quad(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// q6_run16 of a run at byte `off` of a stage.
+__device__ __forceinline__ void q6_lds_run16(const uint8_t *st, uint32_t off, uint32_t (&w)[4])
+{
+    const uint32_t sh = off & 3u;
+    const uint8_t *b = st + (off - sh);
+    const u32x4 v = *(const u32x4 *)b;
+    const uint32_t e = *(const uint32_t *)(b + 16);
+    w[0] = __builtin_amdgcn_alignbyte(v.y, v.x, sh);
+    w[1] = __builtin_amdgcn_alignbyte(v.z, v.y, sh);
+    w[2] = __builtin_amdgcn_alignbyte(v.w, v.z, sh);
+    w[3] = __builtin_amdgcn_alignbyte(e, v.w, sh);
+}
+
+__global__ __launch_bounds__(64 * kQ6Waves) void gemv_q6_k3_k(float *dst, const uint8_t *M, const float *v, int out,
+                                                              int in)
+{
+    constexpr int R = kQ6Rows;
+    extern __shared__ __align__(16) uint8_t q6_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int nsb = in / 256, ntask = nsb * 4, npass = (nsb + 15) / 16;
+    const int64_t row_bytes = (int64_t)nsb * 210;
+    uint4 *lx = (uint4 *)q6_lds;  // [slice][high, middle, low plane, sums and scale][ntask]
+    uint8_t *stage = q6_lds + nsb * 1024 + wave * (R * kQ6Stage);
+    const int ngroup = (out + R - 1) / R, step = (int)gridDim.x * kQ6Waves;
+    int grp = (int)blockIdx.x * kQ6Waves + wave, pass = 0;
+
+    uint4 pw[R][kQ6Loads];
+    auto fetch = [&](int g, int p) {
+#pragma unroll
+        for (int rr = 0; rr < R; rr++) {
+            // rows past the end repeat the last; groups past the end read nothing
+            const uintptr_t at = (uintptr_t)M + (int64_t)min(g * R + rr, out - 1) * row_bytes + (int64_t)p * kQ6Run;
+            const int n = min(kQ6Run, (nsb - 16 * p) * 210) + (int)(at & 15u);
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(at & ~(uintptr_t)15), (short)0, g < ngroup ? (n + 3) & ~3 : 0, kRawBufWord3);
+#pragma unroll
+            for (int i = 0; i < kQ6Loads; i++)
+                pw[rr][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, 16 * lane, 1024 * i, 0));
+        }
+    };
+    fetch(grp, 0);
+    // Float4 k4 of the activations: task (k4 / 64) * 4 + (half, slice), slice
+    // j, dword c of each plane; a lane quad holds a group of 16.
+    for (int k4 = threadIdx.x; k4 < nsb * 64; k4 += 64 * kQ6Waves) {
+        const int t = (k4 >> 6) * 4 + ((k4 >> 5) & 1) * 2 + ((k4 >> 2) & 1), j = (k4 >> 3) & 3, c = k4 & 3;
+        const float4 x = ((const float4 *)v)[k4];
+        float am = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
+        const bool bad = !((x.x - x.x) + (x.y - x.y) + (x.z - x.z) + (x.w - x.w) == 0.f);
+        if (bad) am = INFINITY;
+        am = fmaxf(am, q6_quad<0xB1>(am));
+        am = fmaxf(am, q6_quad<0x4E>(am));
+        float dx = am * (1.f / 8323072.f), inv = 8323072.f / am;
+        int k = 0;
+        if (am < 1e-30f) {  // the reciprocal's range: a power of two instead
+            int ea = 0;
+            (void)frexpf(am, &ea);
+            k = am > 0.f ? min(22 - ea, 145) : 0;
+            inv = 1.f;
+            dx = ldexpf(1.f, -k);
+        }
+        if (am == INFINITY) {  // infinities and NaN anywhere in a row make its result NaN
+            inv = 0.f;
+            dx = __builtin_nanf("");
+        }
+        const float xv[4] = {x.x, x.y, x.z, x.w};
+        uint32_t ph = 0, pm = 0, pl = 0;
+        int sh = 0, sm = 0, sl = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int xi = am == INFINITY ? 0 : (int)rintf(ldexpf(xv[q], k) * inv);
+            const int l = (int)(int8_t)xi, m8 = (xi - l) >> 8, m = (int)(int8_t)m8, h = (m8 - m) >> 8;
+            ph |= (uint32_t)(uint8_t)h << (8 * q);
+            pm |= (uint32_t)(uint8_t)m << (8 * q);
+            pl |= (uint32_t)(uint8_t)l << (8 * q);
+            sh += h;
+            sm += m;
+            sl += l;
+        }
+        sh += __float_as_int(q6_quad<0xB1>(__int_as_float(sh)));
+        sh += __float_as_int(q6_quad<0x4E>(__int_as_float(sh)));
+        sm += __float_as_int(q6_quad<0xB1>(__int_as_float(sm)));
+        sm += __float_as_int(q6_quad<0x4E>(__int_as_float(sm)));
+        sl += __float_as_int(q6_quad<0xB1>(__int_as_float(sl)));
+        sl += __float_as_int(q6_quad<0x4E>(__int_as_float(sl)));
+        uint32_t *o = (uint32_t *)(lx + (4 * j) * ntask + t) + c;
+        o[0] = ph;
+        o[4 * ntask] = pm;
+        o[8 * ntask] = pl;
+        o[12 * ntask] = c == 0 ? (uint32_t)(-32 * sh) : c == 1 ? (uint32_t)(-32 * sm) : c == 2 ? (uint32_t)(-32 * sl) : __float_as_uint(dx);
+    }
+    __syncthreads();
+    float acc[R];
+#pragma unroll
+    for (int rr = 0; rr < R; rr++) acc[rr] = 0.f;
+    while (grp < ngroup) {
+        uint32_t ph[R];
+#pragma unroll
+        for (int rr = 0; rr < R; rr++) {
+            ph[rr] = (uint32_t)(((uintptr_t)M + (int64_t)min(grp * R + rr, out - 1) * row_bytes + (int64_t)pass * kQ6Run) & 15u);
+#pragma unroll
+            for (int i = 0; i < kQ6Loads; i++)
+                if (64 * (i + 1) <= kQ6Pieces || lane + 64 * i < kQ6Pieces)
+                    *(uint4 *)(stage + rr * kQ6Stage + 16 * (lane + 64 * i)) = pw[rr][i];
+        }
+        const bool done = pass + 1 == npass;  // of this group
+        const int ng = done ? grp + step : grp, np = done ? 0 : pass + 1;
+        fetch(ng, np);
+        const int t = pass * 64 + lane;
+        if (t < ntask) {
+            const uint32_t b = (uint32_t)lane >> 2, h = ((uint32_t)lane >> 1) & 1u;
+            const int sl = lane & 1;
+            Q6Task w[R];
+#pragma unroll
+            for (int rr = 0; rr < R; rr++) {
+                const uint8_t *st = stage + rr * kQ6Stage;
+                const uint32_t o = ph[rr] + 210u * b;
+                q6_lds_run16(st, o + 64 * h + 16 * sl, w[rr].qa);
+                q6_lds_run16(st, o + 64 * h + 32 + 16 * sl, w[rr].qb);
+                q6_lds_run16(st, o + 128 + 32 * h + 16 * sl, w[rr].qh);
+                const uint32_t os = o + 192 + 8 * h, sh = os & 3u;
+                const uint32_t *sp = (const uint32_t *)(st + (os - sh));
+                w[rr].sc0 = __builtin_amdgcn_alignbyte(sp[1], sp[0], sh);
+                w[rr].sc1 = __builtin_amdgcn_alignbyte(sp[2], sp[1], sh);
+                w[rr].d = half_bits_to_float(*(const uint16_t *)(st + o + 208));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint4 xh = lx[(4 * j) * ntask + t], xm = lx[(4 * j + 1) * ntask + t], xl = lx[(4 * j + 2) * ntask + t],
+                            xs = lx[(4 * j + 3) * ntask + t];
+                const int shq = 4 * (j >> 1);
+                // sc[8h + 16s/16 + 2j]: byte s + 2j of the half's 8
+                const int k = sl + 2 * j;
+#pragma unroll
+                for (int rr = 0; rr < R; rr++) {
+                    const uint32_t *ql = (j & 1) ? w[rr].qb : w[rr].qa;
+                    int sh = (int)xs.x, sm = (int)xs.y, so = (int)xs.z;
+                    const uint32_t ah[4] = {xh.x, xh.y, xh.z, xh.w}, am[4] = {xm.x, xm.y, xm.z, xm.w}, al[4] = {xl.x, xl.y, xl.z, xl.w};
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const uint32_t hb = j < 2 ? w[rr].qh[c] << (4 - 2 * j) : w[rr].qh[c] >> (2 * j - 4);
+                        const int q = (int)(((ql[c] >> shq) & 0x0F0F0F0Fu) | (hb & 0x30303030u));
+                        sh = __builtin_amdgcn_sdot4(q, (int)ah[c], sh, false);
+                        sm = __builtin_amdgcn_sdot4(q, (int)am[c], sm, false);
+                        so = __builtin_amdgcn_sdot4(q, (int)al[c], so, false);
+                    }
+                    const uint32_t scw = k < 4 ? w[rr].sc0 : w[rr].sc1;
+                    const float sc = (float)(int8_t)(scw >> (8 * (k & 3)));
+                    const float sx = fmaf((float)sh, 65536.f, (float)(sm * 256 + so));
+                    acc[rr] = fmaf(w[rr].d * sc, sx * __uint_as_float(xs.w), acc[rr]);
+                }
+            }
+        }
+        if (done) {
+#pragma unroll
+            for (int rr = 0; rr < R; rr++) {
+                const float s = wave_reduce_sum(acc[rr]);
+                if (lane == 0 && grp * R + rr < out) dst[grp * R + rr] = s;
+                acc[rr] = 0.f;
+            }
+        }
+        grp = ng;
+        pass = np;
+    }
+}
+
 // Rows per wave: the most (of 4, 2, 1) that still give two workgroups per CU
 // (MI355X: 4 rows at 32000 and 11008 rows, 2 at 4096).  HOLO_Q6K_ROWS=1|2|4
 // forces a value.
@@ -1619,9 +1814,28 @@ void cuda_matmul_q6_k(float *dst, const void *M, const float *v, int out_dim, in
         HOLO_LAUNCH_CHECK();
         return;
     }
+    const uint8_t *W = (const uint8_t *)M;
+    // Through LDS where every wave has two groups of rows or more to stage
+    // under each other (us, straight loads / staged: 32000 x 4096 30.3 / 26.0,
+    // 28000 x 8192 51.5 / 41.0, 8192 x 14336 28.2 / 25.4, 16400 x 4096 16.1 /
+    // 16.0; with less the conversion shows: 8000 x 4096 9.5 / 10.7, 4096 x 4096
+    // 6.0 / 7.4), two workgroups per CU where their LDS fits.  Other activation
+    // modes keep fp32 activations.
+    const size_t lds = (size_t)(in_dim / 256) * 1024 + (size_t)kQ6Waves * kQ6Rows * kQ6Stage;
+    const int wgs = (lds <= 80 * 1024 ? 2 : 1) * num_cus();
+    if (lds <= 160 * 1024 && out_dim >= 2 * kQ6Rows * kQ6Waves * wgs && gemv_default_mode()) {
+        static const hipError_t attr = hipFuncSetAttribute((const void *)gemv_q6_k3_k,
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (attr != hipSuccess) {
+            HOLO_CHECK(attr);
+            return;
+        }
+        launch_timed(gemv_q6_k3_k, dim3(wgs), dim3(64 * kQ6Waves), lds, dst, W, v, out_dim, in_dim);
+        HOLO_LAUNCH_CHECK();
+        return;
+    }
     const int R = q6_rows_per_wave(out_dim);
     const dim3 grid((out_dim + 4 * R - 1) / (4 * R));
-    const uint8_t *W = (const uint8_t *)M;
     if (R == 4)
         launch_timed(gemv_q6_k2_k<4>, grid, dim3(256), 0, dst, W, v, out_dim, in_dim);
     else if (R == 2)
