@@ -97,3 +97,34 @@ def test_decode_step_rotation(holo, synth, hd, nh, nkv, pos):
     lib.cuda_sync()
     holo.check("op by op")
     assert normwise_err(down(logits, vocab), down(want, vocab)) <= 5e-6
+
+
+@pytest.mark.parametrize("low", [np.float32(-3e14), np.float32(-np.inf)], ids=["finite", "infinite"])
+@pytest.mark.parametrize("hd,nh,nkv,kv_len,first", [(128, 2, 1, 1, 0), (128, 4, 2, 40, 40), (64, 4, 2, 300, 130),
+                                                    (128, 32, 32, 600, 600), (128, 32, 32, 600, 75),
+                                                    (128, 1, 1, 9001, 3000), (4, 2, 1, 8193, 5000)])
+def test_decode_very_low_scores(holo, synth, hd, nh, nkv, kv_len, first, low):
+    """Scores below -1e30 (or of minus infinity) in the first `first`
+    positions, zero in the others: the values of the others are averaged, or
+    of all positions where every score is the same low one.  A position of
+    minus infinity counts nothing, so some position is finite there."""
+    print(f"case low scores hd {hd} heads {nh}/{nkv} kv_len {kv_len} first {first} low {low}", flush=True)
+    if np.isinf(low):
+        first = min(first, kv_len - 1)
+    lib = holo.lib()
+    kv_dim = nkv * hd
+    q = np.full(nh * hd, np.float32(3e14))
+    kc = np.zeros((kv_len, kv_dim), np.float32)
+    kc[:first] = low
+    vc = synth.normal(kv_len * kv_dim, seed=45)
+    d = holo.DeviceBuffer(4 * nh * hd)
+    dq, dk, dv = up(holo, q), up(holo, kc), up(holo, vc)
+    lib.cuda_multi_head_attention(d.ptr, dq.ptr, dk.ptr, dv.ptr, kv_len, hd, nh, nkv)
+    lib.cuda_sync()
+    holo.check("low scores")
+    V = vc.reshape(kv_len, nkv, hd).astype(np.float64)
+    counted = V[first:] if first < kv_len else V
+    want = np.repeat(counted.mean(0), nh // nkv, axis=0).reshape(-1)
+    # equal weights are exact, so only the sums of values round: their terms
+    # are N(0, 1), their mean N(0, 1) / sqrt(n)
+    assert np.max(np.abs(down(d, nh * hd) - want)) <= 8 * 2.0**-24
