@@ -31,8 +31,10 @@ namespace holo {
 // scale from all of it and splits and stores float4s part * blockIdx.y ..
 // of it (part a multiple of 8 and at most NT), which it loads a second time.
 // The row's largest |silu(g) u| comes from the hardware's exp2 and reciprocal
-// (off by |g| 2^-23 and a few ulp: under 2^-16 up to |g| = 88, where silu ends);
-// where that could change the power of two, it is found again with expf.
+// (off by |g| 2^-23 and a few ulp: under 2^-16 down to g = -87; from -87.3 on
+// the reciprocal is subnormal and comes out as zero, where silu goes on to
+// -88.7); where that could change the power of two, or some g of the row lies
+// below -87, it is found again with expf.
 namespace {
 enum XSplitMode { XS_PLAIN = 0, XS_SWIGLU = 1, XS_NORM = 2 };
 
@@ -78,10 +80,11 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         if constexpr (MODE == XS_NORM)
             pw = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
     }
-    float ss = 0.f;
+    float ss = 0.f, gmin = 0.f;
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         if constexpr (MODE == XS_SWIGLU && PART) {
+            gmin = fminf(gmin, fminf(fminf(v[j].x, v[j].y), fminf(v[j].z, v[j].w)));
             auto sg = [](float g) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504f)); };
             v[j] = make_float4(sg(v[j].x) * wv[j].x, sg(v[j].y) * wv[j].y, sg(v[j].z) * wv[j].z, sg(v[j].w) * wv[j].w);
         } else if constexpr (MODE == XS_SWIGLU) {
@@ -109,9 +112,10 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         }
         am = fmaxf(am, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
     }
+    if (MODE == XS_SWIGLU && PART && gmin < -87.0f) am = INFINITY;
     am = block_reduce<true>(am, red);
     if constexpr (MODE == XS_SWIGLU && PART) {
-        // within 2^-15 of a power of two, tiny (the reciprocal flushes), or not finite
+        // within 2^-15 of a power of two, tiny, not finite or a g below -87
         if (((__float_as_uint(am) + 256u) & 0x7FFFFFu) < 512u || am < 1e-30f) {
             am = 0.f;
             for (int j = 0; j < NV; j++) {

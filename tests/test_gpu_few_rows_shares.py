@@ -43,3 +43,28 @@ def test_few_rows_shares(holo, synth, oracle, t, M, K):
     holo.check("shared rows")
     check_rows(down(dY, M * N).reshape(M, N), X, w, np.arange(M), t, K)
     assert np.array_equal(down(dZ, M * N), 0.0 + down(dT, M * N), equal_nan=True)
+
+
+@pytest.mark.parametrize("M,K", [(3, 1056), (23, 11008), (85, 4096)])
+def test_few_rows_shares_end_of_silu(holo, synth, oracle, M, K):
+    """Ordinary rows whose largest silu(g) u is at a g where 1 / (1 + e^-g) is
+    subnormal, as u is huge there: the row's scale has to come from it."""
+    print(f"case end of silu {M}x{K}", flush=True)
+    lib = holo.lib()
+    N = 40
+    src, w = weights(synth, oracle, Q8_0, N, K, seed=M + K)
+    G = synth.normal(M * K, seed=K + 2).reshape(M, K)
+    U = synth.normal(M * K, seed=K + 3).reshape(M, K)
+    for r, (g, u) in enumerate([(-88.0, 1e38), (-87.4, -3e38), (-88.6, 2e38)]):
+        G[r, K // 3 + r], U[r, K // 3 + r] = g, u
+    dW, dG, dU, dR = up(holo, src), up(holo, G), up(holo, U), up(holo, np.zeros(M * N, np.float32))
+    dT, dZ, dH = (holo.DeviceBuffer(4 * n) for n in (M * N, M * N, M * K))
+    lib.cuda_silu_mul(dH.ptr, dG.ptr, dU.ptr, M * K)
+    lib.holo_matmul_batch(dT.ptr, dW.ptr, dH.ptr, M, N, K, Q8_0)
+    lib.holo_matmul_batch_swiglu_add(dZ.ptr, dW.ptr, dG.ptr, dU.ptr, dR.ptr, M, N, K, Q8_0)
+    lib.cuda_sync()
+    holo.check("end of silu")
+    H = down(dH, M * K).reshape(M, K)
+    assert all(np.max(np.abs(H[r])) > 20 for r in range(3))
+    check_rows(down(dZ, M * N).reshape(M, N), H, w, np.arange(M), Q8_0, K)
+    assert np.array_equal(down(dZ, M * N), 0.0 + down(dT, M * N))
