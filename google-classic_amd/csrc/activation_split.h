@@ -24,9 +24,11 @@ namespace holo {
 // 32-block is the 8 float4 of 8 adjacent lanes (K % 32 == 0); Sx holds the
 // block sums of the scaled values (for the Q4_K min term).
 // OPS: the halves in the operand order of few_rows.hip instead, and Sx as
-// [rows / 16][block][16]; n_zero counters at `zero` are cleared.  There the
-// low half of an infinite value is zero, so that the products of a row with
-// infinities are the infinities (and NaNs) that fp32 gives.
+// [rows / 16][block][16]; n_zero counters at `zero` are cleared.  Two halves
+// cannot hold a row with infinities (an infinity's low half is a NaN, its
+// block sum meets the min term's infinity, its neighbours have no common
+// scale): such a row leaves its fp32 values in the place of its operands, and
+// Rs = -1 tells the product to take it from them.
 // PART (with OPS): gridDim.y workgroups share a row: each finds the row's
 // scale from all of it and splits and stores float4s part * blockIdx.y ..
 // of it (part a multiple of 8 and at most NT), which it loads a second time.
@@ -128,6 +130,7 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
             am = block_reduce<true>(am, red);
         }
     }
+    const bool raw = OPS && am == INFINITY;
     // 2^e with a * 2^e in [2^14, 2^15); e = 0 for a zero or non-finite row
     int e = 0;
     if (am > 0.f && am <= 3.4028235e38f) {
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         (void)frexpf(am, &ea);  // am = f * 2^ea, f in [0.5, 1)
         e = 15 - ea;
     }
-    if (threadIdx.x == 0 && (!PART || blockIdx.y == 0)) Rs[blockIdx.x] = ldexpf(1.0f, -e);
+    if (threadIdx.x == 0 && (!PART || blockIdx.y == 0)) Rs[blockIdx.x] = raw ? -1.0f : ldexpf(1.0f, -e);
     if (OPS && blockIdx.x == 0 && (!PART || blockIdx.y == 0))
         for (int j = threadIdx.x; j < n_zero; j += NT) zero[j] = 0;
     if constexpr (PART) {
@@ -159,7 +162,6 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         for (int q = 0; q < 4; q++) {
             h[q] = (_Float16)y[q];
             l[q] = (_Float16)(y[q] - (float)h[q]);
-            if (OPS && fabsf(y[q]) > 65504.0f) l[q] = (_Float16)0.0f;
         }
         // the block's sum over its 8 lanes (octets are wholly live or dead)
         float s = (y[0] + y[1]) + (y[2] + y[3]);
@@ -178,7 +180,8 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
             if (PART ? mine : i < n4) {
                 const int64_t b = (int64_t)(blockIdx.x >> 4) * (n4 >> 3) + (i >> 3);
                 const int m = blockIdx.x & 15;
-                ((uint4 *)Ah)[b * 128 + m + 16 * (i & 3) + (up ? 64 : 0)] = up ? make_uint4(t0, t1, l0, l1) : make_uint4(h0, h1, t0, t1);
+                ((uint4 *)Ah)[b * 128 + m + 16 * (i & 3) + (up ? 64 : 0)] =
+                    raw ? __builtin_bit_cast(uint4, x) : up ? make_uint4(t0, t1, l0, l1) : make_uint4(h0, h1, t0, t1);
                 if (Sx && (i & 7) == 0) Sx[b * 16 + m] = s;
             }
         } else if (i < n4) {

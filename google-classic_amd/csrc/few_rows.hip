@@ -380,6 +380,67 @@ __device__ __forceinline__ v4u fr_operand(const FrOps<WF> &o, int i)
     return w;
 }
 
+// Weights 4i .. 4i + 3 of block b of a row, dequantised.
+template <int WF>
+__device__ __forceinline__ float4 fr_weights(const uint8_t *row, int b, int i)
+{
+    auto four = [](const uint8_t *p) {  // at a 2-byte-aligned address
+        return (uint32_t)((const uint16_t *)p)[0] | (uint32_t)((const uint16_t *)p)[1] << 16;
+    };
+    uint32_t q;
+    float d, off, mn = 0.f;
+    if constexpr (WF == EW_Q4_0) {
+        const uint8_t *p = row + 18 * (int64_t)b;
+        d = half_bits_to_float(*(const uint16_t *)p);
+        q = (four(p + 2 + 4 * (i & 3)) >> (i & 4)) & 0x0F0F0F0Fu;
+        off = 8.f;
+    } else if constexpr (WF == EW_Q8_0) {
+        const uint8_t *p = row + 34 * (int64_t)b;
+        d = half_bits_to_float(*(const uint16_t *)p);
+        q = four(p + 2 + 4 * i) ^ 0x80808080u;
+        off = 128.f;
+    } else if constexpr (WF == EW_Q4_K) {
+        const uint8_t *p = row + 144 * (int64_t)(b >> 3);
+        const v4u h = *(const v4u *)p;
+        uint32_t sc, m;
+        q4_k_scale_min(h.y, h.z, h.w, (uint32_t)b & 7u, sc, m);
+        d = half_bits_to_float(h.x) * (float)sc;
+        mn = half_bits_to_float(h.x >> 16) * (float)m;
+        q = (*(const uint32_t *)(p + 16 + 16 * (b & 7) + 4 * (i & 3)) >> (i & 4)) & 0x0F0F0F0Fu;
+        off = 0.f;
+    } else if constexpr (WF == EW_Q6_K) {
+        const uint8_t *p = row + 210 * (int64_t)(b >> 3);
+        const int h = (b >> 2) & 1, j = b & 3;
+        d = half_bits_to_float(*(const uint16_t *)(p + 208)) * (float)(int8_t)p[192 + 8 * h + 2 * j + (i >> 2)];
+        q = ((four(p + 64 * h + 32 * (j & 1) + 4 * i) >> (4 * (j >> 1))) & 0x0F0F0F0Fu) |
+            ((four(p + 128 + 32 * h + 4 * i) >> (2 * j)) & 0x03030303u) << 4;
+        off = 32.f;
+    } else {
+        const v2u w = *(const v2u *)(row + 64 * (int64_t)b + 8 * i);
+        return make_float4(half_bits_to_float(w.x), half_bits_to_float(w.x >> 16), half_bits_to_float(w.y),
+                           half_bits_to_float(w.y >> 16));
+    }
+    return make_float4(d * ((float)(q & 255u) - off) - mn, d * ((float)((q >> 8) & 255u) - off) - mn,
+                       d * ((float)((q >> 16) & 255u) - off) - mn, d * ((float)(q >> 24) - off) - mn);
+}
+
+// Row m of the activations, left as fp32 values in the place of its operands
+// (xsplit_row_k), times a weight row: a wave, lane l blocks l, l + 64, ...
+template <int WF>
+__device__ __forceinline__ float fr_dot(const uint8_t *row, const uint8_t *A, int m, int nb, int lane)
+{
+    float s = 0.f;
+    for (int b = lane; b < nb; b += 64) {
+        const float4 *x = (const float4 *)(A + ((int64_t)(m >> 4) * nb + b) * 2048) + (m & 15);
+#pragma unroll 1
+        for (int i = 0; i < 8; i++) {
+            const float4 v = x[16 * (i & 3) + 64 * (i >> 2)], w = fr_weights<WF>(row, b, i);
+            s = fmaf(w.w, v.w, fmaf(w.z, v.z, fmaf(w.y, v.y, fmaf(w.x, v.x, s))));
+        }
+    }
+    return wave_reduce_sum(s);
+}
+
 __device__ __forceinline__ v4f mfma_k32(v4u a, v4u b, v4f c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
@@ -656,12 +717,26 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
             rs[r] = a.Rs[m];
             rv[r] = a.R ? a.R[(int64_t)m * Nm + min(n, Nm - 1)] : 0.f;
         }
+        bool raw = false;
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (m0 + r < a.M && n < Nm) {
+        for (int r = 0; r < 4; r++) {
+            raw = raw || (m0 + r < a.M && n < Nm && rs[r] < 0.f);
+            if (m0 + r < a.M && n < Nm && !(rs[r] < 0.f)) {
                 const float y = v[i][r] * rs[r];  // a power of two: exact
                 Ym[(int64_t)(m0 + r) * Nm + n] = a.R ? rv[r] + y : y;
             }
+        }
+        // rows that the halves do not hold: fp32 products, an output at a time
+        for (uint64_t todo = __ballot(raw); todo; todo &= todo - 1) {
+            const int l = __builtin_ctzll(todo), nn = nl + 16 * (t % CT) + (l & 15);
+            for (int r = 0; r < 4; r++) {
+                const int m = (rt0 + t / CT) * 16 + 4 * (l >> 4) + r;
+                if (m >= a.M || !(a.Rs[m] < 0.f)) continue;
+                const float y = fr_dot<WF>(Wm + (int64_t)nn * rowb, a.A, m, nb, lane);
+                const int64_t at = (int64_t)m * Nm + nn;
+                if (lane == 0) Ym[at] = a.R ? a.R[at] + y : y;
+            }
+        }
     }
 }
 

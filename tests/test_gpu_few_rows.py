@@ -180,3 +180,49 @@ def test_few_rows_infinities(holo, synth, oracle):
     assert np.array_equal(outs[0][rest], outs[1][rest])
     want = np.where(w[:, 100] > 0, np.inf, np.where(w[:, 100] < 0, -np.inf, np.nan))
     assert np.array_equal(outs[1][3], want, equal_nan=True)
+
+
+@pytest.mark.parametrize("t,M,N,K", [(Q4_0, 5, 40, 288), (Q4_0, 20, 100, 4096), (Q8_0, 3, 33, 32), (Q8_0, 63, 50, 1056),
+                                     (Q4_K, 7, 70, 256), (Q4_K, 40, 4096, 2304), (Q6_K, 16, 47, 768), (Q6_K, 33, 129, 4096),
+                                     (F16, 5, 31, 288), (F16, 40, 2000, 2080), (F16, 16, 129, 11008)],
+                         ids=lambda v: NAMES[v] if v in NAMES and v != 16 and v != 32 else str(v))
+def test_few_rows_rows_with_infinities(holo, synth, oracle, t, M, N, K):
+    """Rows with infinities anywhere (the last block of a K that is no multiple
+    of 256 among the places), beside finite values past f16's range, give the
+    infinities and NaNs of the dequantised weights' products; the other rows
+    keep their bits, and the add in the store and the SwiGLU in the split give
+    what the unfused sequence gives."""
+    print(f"case infinities {NAMES[t]} {M}x{N}x{K}", flush=True)
+    lib = holo.lib()
+    src, w = weights(synth, oracle, t, N, K, seed=M + N + K)
+    X = synth.normal(M * K, seed=K + 15).reshape(M, K)
+    U = synth.normal(M * K, seed=K + 16).reshape(M, K)
+    R = synth.normal(M * N, seed=K + 17).reshape(M, N)
+    dW, dU, dR = up(holo, src), up(holo, U), up(holo, R)
+    dX, dY = up(holo, X), holo.DeviceBuffer(4 * M * N)
+    lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, t)
+    lib.cuda_sync()
+    y0 = down(dY, M * N).reshape(M, N)
+    X[0, K - 1] = np.inf
+    X[0, K // 2] = 7e4
+    X[M // 2, K - 20] = -np.inf
+    X[M - 1, 3], X[M - 1, K - 2] = np.inf, -np.inf
+    X[M - 1, K // 2] = 1e36  # its products with weights up to 1e2 stay in fp32 range
+    bad = sorted({0, M // 2, M - 1})
+    dX, dS, dZ, dT, dH = up(holo, X), up(holo, R), *(holo.DeviceBuffer(4 * n) for n in (M * N, M * N, M * K))
+    lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, t)
+    lib.holo_matmul_batch_add(dS.ptr, dW.ptr, dX.ptr, dS.ptr, M, N, K, t)
+    lib.cuda_silu_mul(dH.ptr, dX.ptr, dU.ptr, M * K)
+    lib.holo_matmul_batch(dT.ptr, dW.ptr, dH.ptr, M, N, K, t)
+    lib.holo_matmul_batch_swiglu_add(dZ.ptr, dW.ptr, dX.ptr, dU.ptr, dR.ptr, M, N, K, t)
+    lib.cuda_sync()
+    holo.check("rows with infinities")
+    y = down(dY, M * N).reshape(M, N)
+    rest = np.setdiff1d(np.arange(M), bad)
+    assert np.array_equal(y[rest].view(np.uint32), y0[rest].view(np.uint32))
+    with np.errstate(invalid="ignore"):
+        for r in bad:
+            want = (X[r].astype(np.float64) * w).sum(1)  # infinite or NaN each
+            assert np.array_equal(y[r], want.astype(np.float32), equal_nan=True), r
+        assert np.array_equal(down(dS, M * N).reshape(M, N), R + y, equal_nan=True)
+        assert np.array_equal(down(dZ, M * N).reshape(M, N), R + down(dT, M * N).reshape(M, N), equal_nan=True)
