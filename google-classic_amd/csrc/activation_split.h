@@ -27,8 +27,11 @@ namespace holo {
 // [rows / 16][block][16]; n_zero counters at `zero` are cleared.  Two halves
 // cannot hold a row with infinities (an infinity's low half is a NaN, its
 // block sum meets the min term's infinity, its neighbours have no common
-// scale): such a row leaves its fp32 values in the place of its operands, and
-// Rs = -1 tells the product to take it from them.
+// scale), nor, in full, one with a 32-block that lies wholly below a * 2^-17
+// (where the low half runs out of f16's exponents): such a row leaves its fp32
+// values in the place of its operands, and Rs = -1 tells the product to take it
+// from them.  Small blocks count only with `range`: the GEMVs, which few rows
+// would take otherwise, scale every block by itself, the other tiles do not.
 // PART (with OPS): gridDim.y workgroups share a row: each finds the row's
 // scale from all of it and splits and stores float4s part * blockIdx.y ..
 // of it (part a multiple of 8 and at most NT), which it loads a second time.
@@ -38,6 +41,40 @@ namespace holo {
 // -88.7); where that could change the power of two, or some g of the row lies
 // below -87, it is found again with expf.
 namespace {
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float v)
+{
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false)));
+}
+// Maximum over an aligned lane quad, octet, row of 16 and the wave, in every lane of it.
+__device__ __forceinline__ float quad_max(float v) { return max_dpp<0x4E>(max_dpp<0xB1>(v)); }
+__device__ __forceinline__ float octet_max(float v) { return max_dpp<0x141>(quad_max(v)); }  // half mirror
+__device__ __forceinline__ float row_max(float v) { return max_dpp<0x140>(octet_max(v)); }   // mirror
+__device__ __forceinline__ float wave_max(float v)
+{
+    v = row_max(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// Two maxima over a workgroup of 4 or 16 waves, in every thread.  Register
+// permutes and one barrier: with block_reduce's lane shuffles for both, 16 rows
+// of 11008 x 4096 Q4_0 took 15.6 us instead of 14.9.  A second use of the
+// scratch needs a barrier before.
+template <int NW>
+__device__ __forceinline__ float2 block_max2(float a, float b, float2 *scratch)
+{
+    static_assert(NW == 4 || NW == 16);
+    a = wave_max(a);
+    b = wave_max(b);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = make_float2(a, b);
+    __syncthreads();
+    const float2 r = scratch[threadIdx.x & (NW - 1)];
+    return NW == 4 ? make_float2(quad_max(r.x), quad_max(r.y)) : make_float2(row_max(r.x), row_max(r.y));
+}
+
 enum XSplitMode { XS_PLAIN = 0, XS_SWIGLU = 1, XS_NORM = 2 };
 
 template <int NV, int MODE, int NT = 256, bool OPS = false, bool PART = false>
@@ -45,10 +82,11 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
                                                     float *__restrict__ Sx, float *__restrict__ Rs,
                                                     const float *__restrict__ X, const float *__restrict__ U,
                                                     const float *__restrict__ NW, int K, float eps, uint32_t *zero,
-                                                    int n_zero, int part)
+                                                    int n_zero, int part, bool range)
 {
     static_assert(OPS || !PART);
     __shared__ float red[16];
+    __shared__ float2 red2[16];
     const int n4 = K >> 2;
     const int64_t r4 = (int64_t)blockIdx.x * n4;
     // every load of the row issued first, through buffer resources over the
@@ -104,7 +142,25 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
         ss = block_reduce<false>(ss, red);
         scale = 1.0f / sqrtf(ss / (float)K + eps);
     }
-    float am = 0.f;
+    // the row's largest magnitude, and the least of its blocks' (zero blocks aside)
+    float am = 0.f, lo = INFINITY;
+    auto magnitude = [&](const float4 x) {
+        const float m = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
+        am = fmaxf(am, m);
+        if (OPS && range) {
+            const float b = octet_max(m);
+            lo = b > 0.f ? fminf(lo, b) : lo;
+        }
+    };
+    auto reduce = [&]() {
+        if constexpr (OPS) {
+            const float2 r = block_max2<NT / 64>(am, -lo, red2);
+            am = r.x;
+            lo = -r.y;
+        } else {
+            am = block_reduce<true>(am, red);
+        }
+    };
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         if constexpr (MODE == XS_NORM) {
@@ -112,25 +168,27 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
             v[j] = make_float4(v[j].x * scale * w4.x, v[j].y * scale * w4.y, v[j].z * scale * w4.z,
                                v[j].w * scale * w4.w);
         }
-        am = fmaxf(am, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
+        magnitude(v[j]);
     }
     if (MODE == XS_SWIGLU && PART && gmin < -87.0f) am = INFINITY;
-    am = block_reduce<true>(am, red);
+    reduce();
     if constexpr (MODE == XS_SWIGLU && PART) {
         // within 2^-15 of a power of two, tiny, not finite or a g below -87
         if (((__float_as_uint(am) + 256u) & 0x7FFFFFu) < 512u || am < 1e-30f) {
             am = 0.f;
+            lo = INFINITY;
             for (int j = 0; j < NV; j++) {
                 const int o = (int)(threadIdx.x + NT * j) * 16;
                 const float4 g = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
                 const float4 u = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
-                am = fmaxf(am, fmaxf(fmaxf(fabsf((g.x / (1.0f + expf(-g.x))) * u.x), fabsf((g.y / (1.0f + expf(-g.y))) * u.y)),
-                                     fmaxf(fabsf((g.z / (1.0f + expf(-g.z))) * u.z), fabsf((g.w / (1.0f + expf(-g.w))) * u.w))));
+                magnitude(make_float4((g.x / (1.0f + expf(-g.x))) * u.x, (g.y / (1.0f + expf(-g.y))) * u.y,
+                                      (g.z / (1.0f + expf(-g.z))) * u.z, (g.w / (1.0f + expf(-g.w))) * u.w));
             }
-            am = block_reduce<true>(am, red);
+            __syncthreads();
+            reduce();
         }
     }
-    const bool raw = OPS && am == INFINITY;
+    const bool raw = OPS && (am == INFINITY || lo < am * 0x1p-17f);
     // 2^e with a * 2^e in [2^14, 2^15); e = 0 for a zero or non-finite row
     int e = 0;
     if (am > 0.f && am <= 3.4028235e38f) {

@@ -1020,7 +1020,7 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     };
     auto split = [&](auto kern, int nt) {
         hipLaunchKernelGGL(kern, dim3(M, shares), dim3(nt), 0, stream(), (uint2 *)A, (uint2 *)nullptr, Sx, Rs, X, U, NW, K,
-                           eps, cnt, counters, part);
+                           eps, cnt, counters, part, M < 64);
     };
     const bool small = K <= 4096;
     // the normed form keeps rms_norm_rows4_k's 256 threads and summation order

@@ -226,3 +226,48 @@ def test_few_rows_rows_with_infinities(holo, synth, oracle, t, M, N, K):
             assert np.array_equal(y[r], want.astype(np.float32), equal_nan=True), r
         assert np.array_equal(down(dS, M * N).reshape(M, N), R + y, equal_nan=True)
         assert np.array_equal(down(dZ, M * N).reshape(M, N), R + down(dT, M * N).reshape(M, N), equal_nan=True)
+
+
+def without_first_unit(src, w, t, N, K):
+    """The matrix with its first 256 weights of every row (32 for the types of
+    32-weight blocks) zero: their scales and minima cleared."""
+    raw, w, n = np.array(src).view(np.uint8).reshape(N, -1).copy(), w.copy(), 256 if t in (Q4_K, Q6_K) else 32
+    for at, size in {Q4_0: [(0, 2)], Q8_0: [(0, 2)], Q4_K: [(0, 4)], Q6_K: [(208, 2)], F16: [(0, 64)]}[t]:
+        raw[:, at:at + size] = 0
+    w[:, :n] = 0
+    return raw.reshape(-1), w
+
+
+@pytest.mark.parametrize("big", [3e7, 1e12, 1e30])
+@pytest.mark.parametrize("t,M,N,K", [(Q4_0, 3, 40, 1056), (Q4_0, 20, 1000, 11008), (Q8_0, 17, 65, 4096), (Q4_K, 40, 100, 2304),
+                                     (Q6_K, 23, 129, 4096), (Q6_K, 63, 50, 16384), (F16, 16, 77, 1056)],
+                         ids=lambda v: str(v))
+def test_few_rows_range(holo, synth, oracle, t, M, N, K, big):
+    """Rows whose largest value lies far above their other blocks, and meets
+    zero weights: the other blocks keep the bits that a GEMV, which scales
+    them by themselves, gives them."""
+    print(f"case range {NAMES[t]} {M}x{N}x{K} {big}", flush=True)
+    lib = holo.lib()
+    src, w = without_first_unit(*weights(synth, oracle, t, N, K, seed=N + K), t, N, K)
+    X = synth.normal(M * K, seed=K + 25).reshape(M, K)
+    U = synth.normal(M * K, seed=K + 26).reshape(M, K)
+    Y0, H = holo.DeviceBuffer(4 * M * N), holo.DeviceBuffer(4 * M * K)
+    rows = sorted({0, M // 2, M - 1})
+    dW, dU = up(holo, src), up(holo, U)
+    lib.holo_matmul_batch(Y0.ptr, dW.ptr, up(holo, X).ptr, M, N, K, t)
+    lib.cuda_sync()
+    y0 = down(Y0, M * N).reshape(M, N)
+    X[rows, 7] = big
+    dX, dT, dZ = up(holo, X), holo.DeviceBuffer(4 * M * N), up(holo, np.zeros(M * N, np.float32))
+    lib.holo_matmul_batch(Y0.ptr, dW.ptr, dX.ptr, M, N, K, t)
+    lib.cuda_silu_mul(H.ptr, dX.ptr, dU.ptr, M * K)
+    lib.holo_matmul_batch(dT.ptr, dW.ptr, H.ptr, M, N, K, t)
+    lib.holo_matmul_batch_swiglu_add(dZ.ptr, dW.ptr, dX.ptr, dU.ptr, dZ.ptr, M, N, K, t)
+    lib.cuda_sync()
+    holo.check("range")
+    y = down(Y0, M * N).reshape(M, N)
+    rest = np.setdiff1d(np.arange(M), rows)
+    assert np.array_equal(y[rest].view(np.uint32), y0[rest].view(np.uint32))
+    check_rows(y, X, w, np.array(rows), t, K)
+    check_rows(down(dT, M * N).reshape(M, N), down(H, M * K).reshape(M, K), w, np.array(rows), t, K)
+    assert np.array_equal(down(dZ, M * N), 0.0 + down(dT, M * N))
