@@ -605,7 +605,10 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
                             const v4u ah = av[cur][i][m][0], al = av[cur][i][m][1];
                             const v4f zero = {0.f, 0.f, 0.f, 0.f};
                             if constexpr (WF == EW_F16) {
-                                acc[m][j] = mfma_k32(al, w, mfma_k32(ah, w, acc[m][j]));
+                                // a block's two products summed first: all in one chain of products on
+                                // acc, 16 x 4096 x 14336 was off by 3.9e-7 (2-norm), a GEMV a row is by
+                                // 2.8e-7, this by 1.3e-7
+                                acc[m][j] += mfma_k32(ah, w, zero) + mfma_k32(al, w, zero);
                             } else if constexpr (WF == EW_Q6_K) {
                                 const uint32_t sc = ((b & 2) ? o[j].s1 : o[j].s0) >> (16 * (b & 1));
                                 const float sc0 = o[j].d * (float)(int8_t)(sc & 0xFFu);
@@ -749,6 +752,11 @@ struct FrPlan {
     float us;  // the estimate
 };
 
+// Column tiles of a workgroup before its registers spill (four of F16: 128 to
+// 216 bytes a lane; three of 64 rows, 92 bytes, still the fastest at 48 x 11008
+// x 4096: 50.6 us, two 56.4).
+constexpr int few_max_ct(int kind, int mt) { return kind == EW_F16 || (kind == EW_Q8_0 && mt == 4) ? 3 : 4; }
+
 // Picks the plan with the least estimated time, fitted to a sweep of mt, ct
 // and ks over 30 shapes of all types, 16 to 400 rows, out 500 to 14336, in
 // 1024 to 14336 (the picks there are within 3% of the best plan).  In us: per
@@ -768,7 +776,7 @@ FrPlan few_plan(int kind, const int *N, int nmat, int M, int nb)
     for (int mt = 1; mt <= 4; mt *= 2) {
         if (mt > 1 && 16 * mt >= 2 * M) break;
         if (mt < 4 && M > 32) continue;
-        for (int ct = 1; ct <= (kind == EW_Q8_0 && mt == 4 ? 3 : 4); ct++) {  // 64 x 64 Q8_0 spills
+        for (int ct = 1; ct <= few_max_ct(kind, mt); ct++) {
             int nct = 0;
             for (int i = 0; i < nmat; i++) nct += (N[i] + 16 * ct - 1) / (16 * ct);
             const int nrt = (M + 16 * mt - 1) / (16 * mt);
@@ -817,10 +825,11 @@ void launch_few_st(const FrArgs &a)
 template <int WF, int MT>
 void launch_few_ct(const FrArgs &a, int ct)
 {
+    constexpr int M = few_max_ct(WF, MT);
     if (ct == 1) launch_few_st<WF, MT, 1>(a);
     else if (ct == 2) launch_few_st<WF, MT, 2>(a);
-    else if (ct == 3 || (WF == EW_Q8_0 && MT == 4)) launch_few_st<WF, MT, 3>(a);
-    else launch_few_st<WF, MT, WF == EW_Q8_0 && MT == 4 ? 3 : 4>(a);
+    else if (ct == 3) launch_few_st<WF, MT, M < 3 ? M : 3>(a);
+    else launch_few_st<WF, MT, M < 4 ? M : 4>(a);
 }
 template <int WF>
 void launch_few_mt(const FrArgs &a, const FrPlan &p)
@@ -934,6 +943,9 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     for (int i = 0; i < nmat; i++) {
         kinds[i] = few_kind(types[i]);
         if (kinds[i] < 0 || !Y[i] || N[i] <= 0) return false;
+        // a GEMV per row: its sums of a short row round less (K = 512: 8.5e-8
+        // normwise, here 9.2e-8; 1024: 1.0e-7 and 9.6e-8)
+        if (kinds[i] == EW_F16 && M < 64 && nb < 32) return false;
         need_sx = need_sx || kinds[i] == EW_Q4_K;
         // 32-bit byte offsets into a matrix
         const int64_t rowb = kinds[i] == EW_Q4_K   ? (int64_t)(nb / 8) * 144

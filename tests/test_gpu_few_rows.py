@@ -271,3 +271,25 @@ def test_few_rows_range(holo, synth, oracle, t, M, N, K, big):
     check_rows(y, X, w, np.array(rows), t, K)
     check_rows(down(dT, M * N).reshape(M, N), down(H, M * K).reshape(M, K), w, np.array(rows), t, K)
     assert np.array_equal(down(dZ, M * N), 0.0 + down(dT, M * N))
+
+
+@pytest.mark.parametrize("t", [Q4_0, Q8_0, Q4_K, Q6_K, F16], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("M,N,K", [(16, 500, 256), (16, 500, 1024), (3, 500, 2048), (16, 1000, 4096), (23, 500, 11008),
+                                   (40, 300, 14336), (63, 4096, 4096)])
+def test_few_rows_no_less_precise_than_gemvs(holo, synth, oracle, t, M, N, K):
+    """The error against 64 bits (2-norm) is no larger than that of the GEMVs,
+    one per row, that these products replace."""
+    print(f"case precision {NAMES[t]} {M}x{N}x{K}", flush=True)
+    lib = holo.lib()
+    src, w = weights(synth, oracle, t, N, K, seed=M + N + K)
+    X = synth.normal(M * K, seed=K + 35).reshape(M, K)
+    dW, dX, dY, dG = up(holo, src), up(holo, X), holo.DeviceBuffer(4 * M * N), holo.DeviceBuffer(4 * M * N)
+    lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, t)
+    for m in range(M):
+        lib.holo_matmul(dG.ptr + 4 * m * N, dW.ptr, dX.ptr + 4 * m * K, N, K, t)
+    lib.cuda_sync()
+    holo.check("precision")
+    truth = X.astype(np.float64) @ w.astype(np.float64).T
+    here, gemv = (np.linalg.norm(down(d, M * N).reshape(M, N) - truth) / np.linalg.norm(truth) for d in (dY, dG))
+    print(f"  {here:.2e}, one GEMV a row {gemv:.2e}", flush=True)
+    assert here <= gemv
