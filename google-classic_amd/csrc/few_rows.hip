@@ -380,6 +380,24 @@ __device__ __forceinline__ v4u fr_operand(const FrOps<WF> &o, int i)
     return w;
 }
 
+// Eight f16 weights with infinities (and NaNs) replaced by the largest finite
+// values, for the low half: a weight's infinity has the high half's product for
+// its sign, and a low half of zero or of the other sign would make it a NaN.
+// As integers: positive values in signed order, negative ones in unsigned
+// (16 x 11008 x 4096 33.9 -> 34.1 us; float minima 35.2).
+__device__ __forceinline__ v4u finite_f16(v4u w)
+{
+    typedef short s2 __attribute__((ext_vector_type(2)));
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t x = w[i];
+        const s2 p = __builtin_elementwise_min(__builtin_bit_cast(s2, x), s2{0x7BFF, 0x7BFF});
+        w[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(us2, p), us2{0xFBFF, 0xFBFF}));
+    }
+    return w;
+}
+
 // Weights 4i .. 4i + 3 of block b of a row, dequantised.
 template <int WF>
 __device__ __forceinline__ float4 fr_weights(const uint8_t *row, int b, int i)
@@ -600,6 +618,8 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
 #pragma unroll
                     for (int j = 0; j < CT; j++) {
                         const v4u w = fr_operand<WF>(o[j], b);
+                        v4u wl = w;
+                        if constexpr (WF == EW_F16) wl = finite_f16(w);
 #pragma unroll
                         for (int m = 0; m < MT; m++) {
                             const v4u ah = av[cur][i][m][0], al = av[cur][i][m][1];
@@ -608,7 +628,7 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
                                 // a block's two products summed first: all in one chain of products on
                                 // acc, 16 x 4096 x 14336 was off by 3.9e-7 (2-norm), a GEMV a row is by
                                 // 2.8e-7, this by 1.3e-7
-                                acc[m][j] += mfma_k32(ah, w, zero) + mfma_k32(al, w, zero);
+                                acc[m][j] += mfma_k32(ah, w, zero) + mfma_k32(al, wl, zero);
                             } else if constexpr (WF == EW_Q6_K) {
                                 const uint32_t sc = ((b & 2) ? o[j].s1 : o[j].s0) >> (16 * (b & 1));
                                 const float sc0 = o[j].d * (float)(int8_t)(sc & 0xFFu);

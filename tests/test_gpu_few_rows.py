@@ -293,3 +293,32 @@ def test_few_rows_no_less_precise_than_gemvs(holo, synth, oracle, t, M, N, K):
     here, gemv = (np.linalg.norm(down(d, M * N).reshape(M, N) - truth) / np.linalg.norm(truth) for d in (dY, dG))
     print(f"  {here:.2e}, one GEMV a row {gemv:.2e}", flush=True)
     assert here <= gemv
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 40, 1056), (17, 500, 4096), (48, 100, 2080), (100, 64, 512)])
+def test_few_rows_infinite_f16_weights(holo, synth, oracle, M, N, K):
+    """Infinite F16 weights: an infinity of the products' sign (NaN against a
+    zero activation, infinities of both signs and a NaN weight) in their
+    outputs, the other outputs' bits unchanged."""
+    print(f"case infinite f16 weights {M}x{N}x{K}", flush=True)
+    lib = holo.lib()
+    src, w = weights(synth, oracle, F16, N, K, seed=M + N)
+    X = synth.normal(M * K, seed=K + 45).reshape(M, K)
+    X[1, K // 2] = 0.0
+    X[2, K // 2] = 0.5  # its low half is zero
+    dX, outs = up(holo, X), []
+    h = np.array(src).view(np.float16).reshape(N, K).copy()
+    for k in range(2):
+        if k:
+            h[5, K // 2], h[9, K - 1], h[20, 3], h[20, 40], h[31, 7] = np.inf, -np.inf, np.inf, -np.inf, np.nan
+        dW, dY = up(holo, h.view(np.uint16)), holo.DeviceBuffer(4 * M * N)
+        lib.holo_matmul_batch(dY.ptr, dW.ptr, dX.ptr, M, N, K, F16)
+        lib.cuda_sync()
+        outs.append(down(dY, M * N).reshape(M, N))
+    holo.check("infinite f16 weights")
+    rest = np.setdiff1d(np.arange(N), [5, 9, 20, 31])
+    assert np.array_equal(outs[0][:, rest].view(np.uint32), outs[1][:, rest].view(np.uint32))
+    with np.errstate(invalid="ignore"):
+        for n in (5, 9, 20, 31):
+            want = (X.astype(np.float64) * h[n].astype(np.float64)).sum(1)
+            assert np.array_equal(outs[1][:, n], want.astype(np.float32), equal_nan=True), n
