@@ -58,9 +58,11 @@ void exact_release();
 // does not take (no scratch, or a matrix too large).
 bool exact_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
                    const float *U, const float *R, int M, int K, const float *NW = nullptr, float eps = 0.f);
-// What the exact product's 64 x 256 tiles take, in us (an estimate), and
-// whether they fill the chip.
-float exact_tiles_us(int type, int N, int M, int nb, bool *full);
+// What the exact product's 64 x 256 tiles take, in us (an estimate; of Q6_K
+// with or without a prepared copy), and whether they fill the chip.
+float exact_tiles_us(int type, int N, int M, int nb, bool prepared, bool *full);
+// A repacked copy of the Q6_K matrix is registered (holo_prefill_prepare).
+bool q6_prepared(const void *W, int N, int K);
 // The same for a few rows (few_rows.hip): whether a row count goes there
 // instead of to one GEMV per row, the product (false: nothing launched), and
 // the release of its scratch (all of it; a stream's, before it is destroyed).

@@ -792,7 +792,8 @@ FrPlan few_plan(int kind, const int *N, int nmat, int M, int nb)
 {
     FrPlan best = {};
     const int nu = (nb + 7) / 8;
-    const float type = kind == EW_Q8_0 ? 1.15f : kind == EW_Q6_K ? 1.39f : kind == EW_Q4_K ? 1.09f : 1.f;
+    // F16: 3.6 times Q4_0's bytes, in 8-byte pieces (192 x 4096 x 11008 132 us, Q4_0 66)
+    const float type = kind == EW_Q8_0 ? 1.15f : kind == EW_Q6_K ? 1.39f : kind == EW_Q4_K ? 1.09f : kind == EW_F16 ? 2.f : 1.f;
     for (int mt = 1; mt <= 4; mt *= 2) {
         if (mt > 1 && 16 * mt >= 2 * M) break;
         if (mt < 4 && M > 32) continue;
@@ -953,75 +954,97 @@ void few_rows_drop_stream(hipStream_t st)
 
 bool few_rows_take(int M) { return M >= kFrMinRows && gemv_default_mode(); }
 
-bool few_rows_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
-                      const float *U, const float *R, int M, int K, const float *NW, float eps)
+namespace {
+
+// What a call runs: one launch per weight kind, over that kind's matrices in
+// order, and the scratch they share (the launches run one after the other).
+struct FrLaunch {
+    FrPlan p;
+    int kind, n, mat[kExactMats];
+};
+struct FrChoice {
+    FrLaunch l[kExactMats];
+    int nl, counters;
+    size_t parts;
+    bool need_sx;
+};
+
+// Whether the few-row tiles take a call, and their plan.  prepared[i]: a
+// repacked copy of matrix i is registered.
+bool few_choose(const int *types, const int *N, const bool *prepared, int nmat, int M, int K, FrChoice &c)
 {
     if (M > kFrMaxRows) return false;
     const int nb = K / 32;
     int kinds[kExactMats];
-    bool need_sx = false;
+    c.nl = c.counters = 0;
+    c.parts = 0;
+    c.need_sx = false;
     for (int i = 0; i < nmat; i++) {
         kinds[i] = few_kind(types[i]);
-        if (kinds[i] < 0 || !Y[i] || N[i] <= 0) return false;
+        if (kinds[i] < 0 || N[i] <= 0) return false;
         // a GEMV per row: its sums of a short row round less (K = 512: 8.5e-8
         // normwise, here 9.2e-8; 1024: 1.0e-7 and 9.6e-8)
         if (kinds[i] == EW_F16 && M < 64 && nb < 32) return false;
-        need_sx = need_sx || kinds[i] == EW_Q4_K;
+        c.need_sx = c.need_sx || kinds[i] == EW_Q4_K;
         // 32-bit byte offsets into a matrix
         const int64_t rowb = kinds[i] == EW_Q4_K   ? (int64_t)(nb / 8) * 144
                              : kinds[i] == EW_Q6_K ? (int64_t)(nb / 8) * 210
                                                    : (int64_t)nb * (kinds[i] == EW_Q4_0 ? 18 : kinds[i] == EW_Q8_0 ? 34 : 64);
         if ((N[i] + 128) * rowb >= (1LL << 31)) return false;
     }
-    // one launch per weight kind, over that kind's matrices in order
-    struct Launch {
-        FrArgs a;
-        FrPlan p;
-        int kind;
-    } launches[kExactMats];
-    int nl = 0, counters = 0;
-    size_t parts = 0;
     bool many = false;
     float here = 7.6f, tiled = 0.f;  // estimates, us (7.6: the split and two launches)
     bool done[kExactMats] = {false, false, false};
     for (int i = 0; i < nmat; i++) {
         if (done[i]) continue;
-        Launch &l = launches[nl++];
-        l.a = {};
+        FrLaunch &l = c.l[c.nl++];
         l.kind = kinds[i];
-        int n = 0;
+        l.n = 0;
+        int n[kExactMats], columns = 0;
+        bool copies = true;
         for (int j = i; j < nmat; j++) {
             if (done[j] || kinds[j] != kinds[i]) continue;
             done[j] = true;
-            l.a.Y[n] = Y[j];
-            l.a.W[n] = (const uint8_t *)W[j];
-            l.a.n[n++] = N[j];
+            columns += N[j];
+            copies = copies && prepared[j];
+            n[l.n] = N[j];
+            l.mat[l.n++] = j;
         }
-        l.p = few_plan(kinds[i], l.a.n, n, M, nb);
+        l.p = few_plan(kinds[i], n, l.n, M, nb);
         here += l.p.us;
         many = many || l.p.rounds > 3;
-        int tiles = 0, columns = 0;
-        for (int j = 0; j < kExactMats; j++) {
-            if (j < n) tiles += (l.a.n[j] + 16 * l.p.ct - 1) / (16 * l.p.ct);
-            l.a.t_end[j] = j < n ? tiles : INT_MAX;
-            columns += j < n ? l.a.n[j] : 0;
-        }
         bool full;
-        tiled += exact_tiles_us(types[i], columns, M, nb, &full);
+        tiled += exact_tiles_us(types[i], columns, M, nb, copies, &full);
         many = many || full;
-        if (l.p.ks > 1) {  // launches run one after the other: they share the parts and the counters
-            parts = std::max(parts, (size_t)l.p.nct * l.p.nrt * l.p.ks * l.p.mt * l.p.ct * 1024);
-            counters = std::max(counters, l.p.nct * l.p.nrt);
+        if (l.p.ks > 1) {
+            c.parts = std::max(c.parts, (size_t)l.p.nct * l.p.nrt * l.p.ks * l.p.mt * l.p.ct * 1024);
+            c.counters = std::max(c.counters, l.p.nct * l.p.nrt);
         }
     }
     // From 64 rows on, the other tiling where it is estimated 6% better (both
     // sides measured on 70 shapes: the taken one is the faster or within 5% for
     // all that are not `full`): 192 x 11008 x 4096 Q4_0 here 59.5 us, there 71.4;
     // 231 x 6825 x 5632 Q6_K 92.3 and 87.1; 1015 x 890 x 4864 Q8_0 71.2 and 59.4.
-    if (M >= 64 && (many || tiled <= 0.94f * here)) return false;
+    return M < 64 || !(many || tiled <= 0.94f * here);
+}
+
+}  // namespace
+
+bool few_rows_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
+                      const float *U, const float *R, int M, int K, const float *NW, float eps)
+{
+    FrChoice c;
+    bool prepared[kExactMats] = {false, false, false};
+    for (int i = 0; i < nmat; i++) {
+        if (!Y[i]) return false;
+        prepared[i] = M >= 64 && types[i] == HOLO_TYPE_Q6_K && q6_prepared(W[i], N[i], K);
+    }
+    if (!few_choose(types, N, prepared, nmat, M, K, c)) return false;
+    const int nb = K / 32, counters = c.counters;
+    const size_t parts = c.parts;
     const int ntm = (M + 15) / 16;
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t ob = up((size_t)ntm * nb * 2048), sb = need_sx ? up((size_t)ntm * nb * 64) : 0, rb = up((size_t)M * 4),
+    const size_t ob = up((size_t)ntm * nb * 2048), sb = c.need_sx ? up((size_t)ntm * nb * 64) : 0, rb = up((size_t)M * 4),
                  cb = up((size_t)counters * 4);
     const size_t total = ob + sb + rb + cb + parts;
     std::unique_lock<std::mutex> lk(g_slot_mu);
@@ -1036,7 +1059,7 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     if (!wsp) return false;
     uint8_t *ws = (uint8_t *)wsp;
     uint8_t *A = ws;
-    float *Sx = need_sx ? (float *)(ws + ob) : nullptr, *Rs = (float *)(ws + ob + sb);
+    float *Sx = c.need_sx ? (float *)(ws + ob) : nullptr, *Rs = (float *)(ws + ob + sb);
     uint32_t *cnt = (uint32_t *)(ws + ob + sb + rb);
     // Few rows leave most CUs idle: four workgroups a row (each of at most
     // `most` float4s) while they fit the CUs.  23 rows, alone -> four -> eight:
@@ -1066,9 +1089,20 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
         small ? split(xsplit_row_k<1, XS_PLAIN, 1024, true, true>, 1024) : split(xsplit_row_k<4, XS_PLAIN, 1024, true, true>, 1024);
     else small ? split(xsplit_row_k<1, XS_PLAIN, 1024, true>, 1024) : split(xsplit_row_k<4, XS_PLAIN, 1024, true>, 1024);
     HOLO_LAUNCH_CHECK();
-    for (int i = 0; i < nl; i++) {
-        FrArgs &a = launches[i].a;
-        const FrPlan &p = launches[i].p;
+    for (int i = 0; i < c.nl; i++) {
+        const FrLaunch &l = c.l[i];
+        const FrPlan &p = l.p;
+        FrArgs a = {};
+        int tiles = 0;
+        for (int j = 0; j < kExactMats; j++) {
+            if (j < l.n) {
+                a.Y[j] = Y[l.mat[j]];
+                a.W[j] = (const uint8_t *)W[l.mat[j]];
+                a.n[j] = N[l.mat[j]];
+                tiles += (a.n[j] + 16 * p.ct - 1) / (16 * p.ct);
+            }
+            a.t_end[j] = j < l.n ? tiles : INT_MAX;
+        }
         a.A = A;
         a.Sx = Sx;
         a.Rs = Rs;
@@ -1080,7 +1114,7 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
         a.items = p.nct * p.ks;
         a.nrt = p.nrt;
         a.ks = p.ks;
-        switch (launches[i].kind) {
+        switch (l.kind) {
         case EW_Q4_0: launch_few_mt<EW_Q4_0>(a, p); break;
         case EW_Q8_0: launch_few_mt<EW_Q8_0>(a, p); break;
         case EW_Q4_K: launch_few_mt<EW_Q4_K>(a, p); break;
@@ -1093,3 +1127,16 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
 }
 
 }  // namespace holo
+
+extern "C" int holo_few_rows_plan(int type, int M, int N, int K, int prepared, int *plan)
+{
+    holo::FrChoice c;
+    const bool copy = prepared != 0;
+    if (!plan || M < holo::kFrMinRows || !holo::exact_ok(type, K, nullptr) || !holo::few_choose(&type, &N, &copy, 1, M, K, c)) return 0;
+    const int kind = c.l[0].kind;
+    plan[0] = c.l[0].p.mt;
+    plan[1] = c.l[0].p.ct;
+    plan[2] = c.l[0].p.ks;
+    plan[3] = kind == holo::EW_Q4_K || kind == holo::EW_Q6_K || (kind != holo::EW_F16 && K % 256 == 0);
+    return 1;
+}

@@ -1436,16 +1436,19 @@ int exact_kind(int type)
 // About what the second tiling takes, us: 20 and a time per
 // stage of the longest range, more where ranges share a CU (Q4_0, measured:
 // 100 x 4096 x 4096 in 41, 192 x 11008 x 4096 in 73, 128 x 4096 x 11008 in 74;
-// 100 x 4096 x 14336 Q4_K in 104, 128 x 4096 x 11008 Q6_K in 107).
+// 100 x 4096 x 14336 Q4_K in 104, 128 x 4096 x 11008 Q6_K in 107).  Q6_K with
+// its repack (5 us at 1024 x 4096, 25 at 14336 x 4096); on a prepared copy 10 us
+// less puts 72 measured shapes on the faster side within 5%, 100 x 14336 x 4096
+// (68 us on the few-row tiles, 59 on these) and 192 (104, 84) among them.
 // `full`: the launch puts both of its workgroups on every CU (above 256 rows,
 // one: 958 x 1427 x 10240 Q8_0 then takes 117, the few-row tiles 140).
-float exact_tiles_us(int type, int N, int M, int nb, bool *full)
+float exact_tiles_us(int type, int N, int M, int nb, bool prepared, bool *full)
 {
     const int ntm = (M + 63) / 64, nct = (N + 255) / 256, nst = (nb + 1) / 2;
     const int gr = x2_ranges(nct, nst, ntm);
     *full = M > 256 ? ntm * gr > num_cus() : ntm * gr >= 2 * num_cus();
     const float stage = type == HOLO_TYPE_Q4_K ? 1.5f : type == HOLO_TYPE_Q6_K ? 2.0f : type == HOLO_TYPE_Q8_0 ? 1.7f : 1.25f;
-    return 20.f + stage * (float)((int64_t)nct * nst) / (float)gr * std::max(1.f, (float)(ntm * gr) / (float)num_cus());
+    return (type == HOLO_TYPE_Q6_K && prepared ? 10.f : 20.f) + stage * (float)((int64_t)nct * nst) / (float)gr * std::max(1.f, (float)(ntm * gr) / (float)num_cus());
 }
 
 bool exact_init()
@@ -1478,6 +1481,11 @@ const void *prepared_q6r(const void *W, int N, int K)
     return it != g_prep.end() && it->second.N == N && it->second.K == K ? it->second.rec : nullptr;
 }
 
+}  // namespace
+
+bool q6_prepared(const void *W, int N, int K) { return prepared_q6r(W, N, K) != nullptr; }
+
+namespace {
 // Frees every registered copy (cuda_cleanup).
 void prepared_release_all()
 {

@@ -148,6 +148,7 @@ _SIGS = {
     "holo_prefill_set_q8_kernel": (None, [_I]),
     "holo_prefill_get_q8_kernel": (_I, []),
     "holo_prefill_get_mode": (_I, []),
+    "holo_few_rows_plan": (_I, [_I, _I, _I, _I, _I, _P]),
     "holo_batched_qkv_norm": (None, [_P, _P, _P, _P, _P, _P, _P, _P, C.c_float, _P, _I, _I, _I, _I]),
     "holo_batched_ffn_gate_up_norm": (None, [_P, _P, _P, _P, _P, C.c_float, _P, _I, _I, _I]),
     "holo_matmul_add": (None, [_P, _P, _P, _P, _I, _I, _I]),

@@ -324,7 +324,8 @@ void holo_matmul_batch_swiglu_add(float *Y, const void *W, float *G, const float
  * [N][K] (N*K bytes, hipMalloc), writes it, waits for it, and keeps it until
  * holo_prefill_release(W): every later exact batched product on W with the
  * same N and K that would repack it (few-row tiles read W as it is) reads the
- * copy, with the same bits as the per-call form.  W
+ * copy, with the same bits as the per-call form when both run the same tiles
+ * (from 64 rows on the choice counts the repack that a copy saves).  W
  * must not change and must not be freed while registered, and a graph
  * captured while W was registered reads the copy: destroy such graphs
  * before releasing W.  Returns 0 (also
@@ -335,6 +336,13 @@ void holo_matmul_batch_swiglu_add(float *Y, const void *W, float *G, const float
  * waits for the library stream.  cuda_cleanup releases every copy.         */
 int holo_prefill_prepare(const void *W, int N, int K, int type);
 void holo_prefill_release(const void *W);
+/* Whether M rows on one matrix [N][K] run the exact product's tiles for few
+ * rows (1) or not (0), in the default modes and on aligned operands; prepared:
+ * W's copy is registered.  plan receives a workgroup's 16-row and 16-column
+ * tiles, the parts of K, and whether the weights are staged through LDS.
+ * Needs no GPU: the choice depends on the shape and the CU count (256 before
+ * cuda_init).                                                               */
+int holo_few_rows_plan(int type, int M, int N, int K, int prepared, int *plan);
 
 #ifdef __cplusplus
 }
