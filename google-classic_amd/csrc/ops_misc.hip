@@ -5,6 +5,8 @@
 // reference inference loop (src/ai/llm_cuda.c) links and runs unchanged.
 // Each follows the arithmetic of the reference kernel it replaces (cited per
 // function); where the reference has a quirk, it is kept and said so.
+#include <float.h>
+
 #include "common.h"
 #include "quant_blocks.h"
 #include "block_reduce.h"
@@ -864,12 +866,6 @@ static float *g_dec_part = nullptr;
 constexpr int kDecThreads = 512;
 constexpr int kDecMaxSplits = 256;
 
-// What scores are taken relative to where the running maximum is mx.  A
-// maximum of minus infinity (no key yet, or all of them masked) stays one, so
-// that any finite score beats it, but the weights are taken relative to 0:
-// relative to it they would be 2^(-inf + inf).
-__device__ __forceinline__ float softmax_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
-
 // Merges a head's ranges with weights 2^(m_s - M), NS of them per round of
 // loads: thread d holds every range's output d, max and sum, so nothing is
 // exchanged and a merge of up to NS ranges waits once.
@@ -893,14 +889,13 @@ __global__ __launch_bounds__(128) void attn_dec_merge_k(float *out, const float 
         float mx = fmaxf(M, m[0]);
 #pragma unroll
         for (int s = 1; s < NS; s++) mx = fmaxf(mx, m[s]);
-        const float ref = softmax_ref(mx);
-        const float c = __builtin_amdgcn_exp2f(M - ref);  // 0 in the first round
+        const float c = __builtin_amdgcn_exp2f(M - mx);  // 0 in the first round
         L *= c;
         a *= c;
         M = mx;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const float w = __builtin_amdgcn_exp2f(m[s] - ref);
+            const float w = __builtin_amdgcn_exp2f(m[s] - M);
             L = fmaf(w, l[s], L);
             a = fmaf(w, o[s], a);
         }
@@ -998,7 +993,10 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
         kn = *(const float4 *)(lk + 4 * c);
         if (g == 0 && h % (a.n_heads / a.n_kv_heads) == 0) *(float4 *)(a.kw + (int64_t)kvh * hd + 4 * c) = kn;
     }
-    float m = -INFINITY, l = 0.f;
+    // The running maximum starts at the lowest finite value: no finite score lies
+    // below it, and a weight relative to it is a number also where a group has
+    // seen no key yet or only ones of minus infinity.
+    float m = -FLT_MAX, l = 0.f;
     float4 o4 = zero;
     auto use = [&](int b, int p0) {
         float sj[J];
@@ -1012,13 +1010,13 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
             sj[j] = p < p_end ? d : -INFINITY;
             mx = fmaxf(mx, sj[j]);
         }
-        const float ref = softmax_ref(mx), corr = __builtin_amdgcn_exp2f(m - ref);
+        const float corr = __builtin_amdgcn_exp2f(m - mx);
         m = mx;
         l *= corr;
         o4 = make_float4(o4.x * corr, o4.y * corr, o4.z * corr, o4.w * corr);
 #pragma unroll
         for (int j = 0; j < J; j++) {
-            const float w = __builtin_amdgcn_exp2f(sj[j] - ref);
+            const float w = __builtin_amdgcn_exp2f(sj[j] - m);
             l += w;
             o4 = make_float4(fmaf(w, v4[b][j].x, o4.x), fmaf(w, v4[b][j].y, o4.y), fmaf(w, v4[b][j].z, o4.z),
                              fmaf(w, v4[b][j].w, o4.w));
@@ -1034,8 +1032,7 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
 #pragma unroll
     for (int off = 32; off >= LPK; off >>= 1) {
         const float m2 = __shfl_xor(m, off, 64), l2 = __shfl_xor(l, off, 64);
-        const float mx = fmaxf(m, m2), ref = softmax_ref(mx);
-        const float w1 = __builtin_amdgcn_exp2f(m - ref), w2 = __builtin_amdgcn_exp2f(m2 - ref);
+        const float mx = fmaxf(m, m2), w1 = __builtin_amdgcn_exp2f(m - mx), w2 = __builtin_amdgcn_exp2f(m2 - mx);
         const float4 r = make_float4(__shfl_xor(o4.x, off, 64), __shfl_xor(o4.y, off, 64), __shfl_xor(o4.z, off, 64),
                                      __shfl_xor(o4.w, off, 64));
         o4 = make_float4(w1 * o4.x + w2 * r.x, w1 * o4.y + w2 * r.y, w1 * o4.z + w2 * r.z, w1 * o4.w + w2 * r.w);
@@ -1053,11 +1050,10 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
         float M = lm[0];
 #pragma unroll
         for (int w = 1; w < W; w++) M = fmaxf(M, lm[w]);
-        const float ref = softmax_ref(M);
         float L = 0.f, r = 0.f;
 #pragma unroll
         for (int w = 0; w < W; w++) {
-            const float e = __builtin_amdgcn_exp2f(lm[w] - ref);
+            const float e = __builtin_amdgcn_exp2f(lm[w] - M);
             L = fmaf(e, ll[w], L);
             r = fmaf(e, lo[w][t], r);
         }
