@@ -29,16 +29,14 @@ int num_cus();
 // Barrier words of the persistent decode-step kernel (gemv_stream.hip).
 bool gemv_stream_init();
 void gemv_stream_release();
-// The decode-attention range partials (16 MiB), allocated once by cuda_init;
-// without them decode attention runs one range per head.
-bool attention_scratch_init();
-void attention_scratch_release();
 // A decode step's attention with its RoPE, for rows that fit it: q and the raw
 // key kx of position pos are rotated on the way in and the key's cache row is
-// written (the value's is there already).
+// written (the value's is there already).  part: the ranges' partials, of the
+// bytes given for kv_len = pos + 1 (0: one range, no partials).
 bool attention_decode_fits(const float *q, const float *kc, const float *vc, int hd);
+size_t attention_decode_part_bytes(int kv_len, int hd, int n_heads);
 void attention_decode_rope(float *dst, const float *q, const float *kx, float *kc, const float *vc, int pos, int hd,
-                           int n_heads, int n_kv_heads, float base);
+                           int n_heads, int n_kv_heads, float base, float *part);
 void panel_workspace_release();  // the batched products' panel buffers (prefill.hip)
 // The batched products' kept workspaces (prefill.hip): slot 0 weight panels,
 // slot 1 activation panels, slot 2 the exact product's split-K partials.  A device buffer of at least `bytes`, grown with
@@ -64,13 +62,10 @@ float exact_tiles_us(int type, int N, int M, int nb, bool prepared, bool *full);
 // A repacked copy of the Q6_K matrix is registered (holo_prefill_prepare).
 bool q6_prepared(const void *W, int N, int K);
 // The same for a few rows (few_rows.hip): whether a row count goes there
-// instead of to one GEMV per row, the product (false: nothing launched), and
-// the release of its scratch (all of it; a stream's, before it is destroyed).
+// instead of to one GEMV per row, and the product (false: nothing launched).
 bool few_rows_take(int M);
 bool few_rows_product(float *const *Y, const void *const *W, const int *types, const int *N, int nmat, const float *X,
                       const float *U, const float *R, int M, int K, const float *NW, float eps);
-void few_rows_release();
-void few_rows_drop_stream(hipStream_t st);
 // The GEMVs run their default activation mode (holo_gemv_set_xmode).
 bool gemv_default_mode();
 // The exact route for nmat matrices of rows RMS-normed on the way in, when

@@ -41,12 +41,12 @@
 #include "quant_blocks.h"
 #include "activation_split.h"
 #include "exact_blocks.h"
+#include "stream_scratch.h"
 
 #include <hip/hip_ext.h>
 #include <algorithm>
 #include <limits.h>
 
-#include <mutex>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -872,85 +872,7 @@ int few_kind(int type)
     }
 }
 
-// Scratch of a call (operands, counters, parts): one kept buffer per stream,
-// so calls on several streams never share one, for up to kFrSlots streams; a
-// further stream takes over the least recently used buffer once the device is
-// idle.  g_slot_mu is held from taking a buffer to the last launch that reads
-// it, so calls of several threads on one stream run one after the other.
-// (Stream-ordered allocations instead cost about 10 us of host time a call.)
-struct FrSlot {
-    hipStream_t stream;
-    int dev;
-    void *buf;
-    size_t bytes;
-    uint64_t used;  // 0: free
-};
-constexpr int kFrSlots = 8;
-std::mutex g_slot_mu;
-FrSlot g_slots[kFrSlots];
-uint64_t g_slot_clock = 0;
-
-// A buffer of at least `bytes` for the library stream; nullptr when there is
-// no memory.  g_slot_mu is held.
-void *few_slot(size_t bytes)
-{
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    FrSlot *s = nullptr, *old = &g_slots[0];
-    for (FrSlot &t : g_slots) {
-        if (t.used && t.stream == stream() && t.dev == dev) s = &t;
-        if (t.used < old->used) old = &t;
-    }
-    if (!s) {
-        s = old;
-        if (s->used && hipDeviceSynchronize() != hipSuccess) return nullptr;
-        if (s->used && s->dev != dev) {  // a buffer of another device
-            (void)hipFree(s->buf);
-            s->buf = nullptr;
-            s->bytes = 0;
-        }
-        s->stream = stream();
-        s->dev = dev;
-    }
-    s->used = ++g_slot_clock;
-    if (s->bytes >= bytes) return s->buf;
-    if (s->buf) {
-        if (hipStreamSynchronize(stream()) != hipSuccess) return nullptr;
-        (void)hipFree(s->buf);
-    }
-    s->buf = nullptr;
-    s->bytes = 0;
-    const size_t grown = std::max(bytes, (size_t)1 << 20);
-    if (hipMalloc(&s->buf, grown) != hipSuccess) {
-        (void)hipGetLastError();
-        s->buf = nullptr;
-        return nullptr;
-    }
-    s->bytes = grown;
-    return s->buf;
-}
-
 }  // namespace
-
-void few_rows_release()
-{
-    std::lock_guard<std::mutex> lk(g_slot_mu);
-    for (FrSlot &s : g_slots) {
-        if (s.buf) (void)hipFree(s.buf);
-        s = FrSlot{};
-    }
-}
-
-void few_rows_drop_stream(hipStream_t st)
-{
-    std::lock_guard<std::mutex> lk(g_slot_mu);
-    for (FrSlot &s : g_slots)
-        if (s.used && s.stream == st) {
-            (void)hipStreamSynchronize(st);
-            if (s.buf) (void)hipFree(s.buf);
-            s = FrSlot{};
-        }
-}
 
 bool few_rows_take(int M) { return M >= kFrMinRows && gemv_default_mode(); }
 
@@ -1047,17 +969,9 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     const size_t ob = up((size_t)ntm * nb * 2048), sb = c.need_sx ? up((size_t)ntm * nb * 64) : 0, rb = up((size_t)M * 4),
                  cb = up((size_t)counters * 4);
     const size_t total = ob + sb + rb + cb + parts;
-    std::unique_lock<std::mutex> lk(g_slot_mu);
-    // under capture a stream-ordered allocation: a graph must not hold a kept buffer
-    const bool own = stream_capturing();
-    void *wsp = nullptr;
-    if (!own) wsp = few_slot(total);
-    else if (hipMallocAsync(&wsp, total, stream()) != hipSuccess) {
-        (void)hipGetLastError();
-        wsp = nullptr;
-    }
-    if (!wsp) return false;
-    uint8_t *ws = (uint8_t *)wsp;
+    const StreamScratch scratch(total);
+    uint8_t *ws = (uint8_t *)scratch.get();
+    if (!ws) return false;
     uint8_t *A = ws;
     float *Sx = c.need_sx ? (float *)(ws + ob) : nullptr, *Rs = (float *)(ws + ob + sb);
     uint32_t *cnt = (uint32_t *)(ws + ob + sb + rb);
@@ -1122,7 +1036,6 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
         default: launch_few_mt<EW_F16>(a, p); break;
         }
     }
-    if (own) HOLO_CHECK(hipFreeAsync(ws, stream()));
     return true;
 }
 

@@ -177,12 +177,14 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
     const int exact = flags & HOLO_FORWARD_EXACT;
     const int64_t layer_cache = (int64_t)m->max_seq * kv_dim;
 
-    // stream-ordered scratch: token ids, x, xb, q, att, hb, hb2, and one raw key
-    // row (otherwise k and v are written straight into the caches)
+    // stream-ordered scratch: token ids, x, xb, q, att, hb, hb2, and for one row
+    // the raw key (otherwise k and v are written straight into the caches) and
+    // the attention's partials
     const size_t rowsz = (size_t)n * sizeof(float);
     const size_t sz_tok = ((size_t)n * sizeof(int) + 255) & ~(size_t)255;
     const size_t sizes[] = {sz_tok, rowsz * dim, rowsz * dim, rowsz * q_dim, rowsz * q_dim, rowsz * ffn, rowsz * ffn,
-                            sizeof(float) * (size_t)kv_dim};
+                            sizeof(float) * (size_t)kv_dim,
+                            n == 1 ? attention_decode_part_bytes(pos0 + 1, hd, m->n_heads) : 0};
     constexpr int kBufs = sizeof(sizes) / sizeof(sizes[0]);
     size_t total = 0;
     for (size_t s : sizes) total += (s + 255) & ~(size_t)255;
@@ -198,7 +200,7 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
     int *dtok = (int *)bufs[0];
     float *x = (float *)bufs[1], *xb = (float *)bufs[2], *q = (float *)bufs[3], *att = (float *)bufs[4];
     float *hb = (float *)bufs[5], *hb2 = (float *)bufs[6];
-    float *kx = (float *)bufs[7];
+    float *kx = (float *)bufs[7], *part = sizes[8] ? (float *)bufs[8] : nullptr;
 
     // embeddings: all n rows in one launch
     HOLO_CHECK(hipMemcpyAsync(dtok, tokens, (size_t)n * sizeof(int), hipMemcpyHostToDevice, stream()));
@@ -229,7 +231,7 @@ int holo_llama_forward(const holo_llama_t *m, const int *tokens, int n, int pos0
             matmul_qkv(q, k, v, L, xb, n, q_dim, kv_dim, dim, exact);
         }
         if (rope1) {
-            attention_decode_rope(att, q, kx, kc, vc, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base);
+            attention_decode_rope(att, q, kx, kc, vc, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base, part);
         } else {
             holo_rope_rows(q, k, n, pos0, hd, m->n_heads, m->n_kv_heads, m->rope_base);  // k rotated in the cache
             holo_attention_prefill(att, q, kc, vc, n, pos0, hd, m->n_heads, m->n_kv_heads);

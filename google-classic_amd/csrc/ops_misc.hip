@@ -10,6 +10,7 @@
 #include "common.h"
 #include "quant_blocks.h"
 #include "block_reduce.h"
+#include "stream_scratch.h"
 
 #include "../../include/holo_forward.h"
 
@@ -861,8 +862,7 @@ static int q6_rows_per_wave(int out_dim)
 // us in all against 13.3 at a large copy's rate and 19.7 before; at 512 the
 // launches and one round trip of loads (range kernel 6.4, merge 2.4 us; before
 // 8.8 and 4.0).
-constexpr size_t kDecPartFloats = (size_t)4 << 20;  // 16 MiB of range partials, allocated by cuda_init
-static float *g_dec_part = nullptr;
+constexpr size_t kDecPartFloats = (size_t)4 << 20;  // 16 MiB of range partials at most
 constexpr int kDecThreads = 512;
 constexpr int kDecMaxSplits = 256;
 
@@ -1085,19 +1085,25 @@ bool attention_decode_fits(const float *q, const float *kc, const float *vc, int
 // x 8 heads: 15 ranges 6.7 us, 30 8.4).
 static int decode_splits(int kv_len, int hd, int n_heads)
 {
-    if (!g_dec_part || (int64_t)kv_len * hd <= 256 * 128) return 1;
+    if ((int64_t)kv_len * hd <= 256 * 128) return 1;
     int want = num_cus() / n_heads;
     if (want > 16) want = max(16, num_cus() / 2 / n_heads);
     want = min(want, min(kDecMaxSplits, (int)(kDecPartFloats / ((size_t)n_heads * (hd + 4)))));
     return max(1, min(want, (kv_len + 63) / 64));
 }
 
+size_t attention_decode_part_bytes(int kv_len, int hd, int n_heads)
+{
+    const int splits = decode_splits(kv_len, hd, n_heads);
+    return splits > 1 ? (size_t)n_heads * splits * (hd + 4) * sizeof(float) : 0;
+}
+
+// a.part: room for the ranges' partials, or nullptr for one range a head.
 static void decode_attention(DecArgs a, bool rope)
 {
-    int splits = decode_splits(a.kv_len, a.hd, a.n_heads);
+    int splits = a.part ? decode_splits(a.kv_len, a.hd, a.n_heads) : 1;
     a.chunk = (a.kv_len + splits - 1) / splits;
     splits = (a.kv_len + a.chunk - 1) / a.chunk;  // every range holds at least one key
-    a.part = g_dec_part;
     auto run = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(splits, a.n_heads), dim3(kDecThreads), 0, stream(), a);
     };
@@ -1113,34 +1119,28 @@ static void decode_attention(DecArgs a, bool rope)
     }
 }
 
+// The partials are the stream's own (or the captured graph's): with one buffer
+// for all, calls under way on two streams would merge each other's.
 static void decode_attention(float *dst, const float *q, const float *kc, const float *vc, int kv_len, int hd,
                              int n_heads, int n_kv_heads)
 {
-    decode_attention(DecArgs{dst, nullptr, q, kc, vc, nullptr, nullptr, kv_len, hd, n_heads, n_kv_heads, 0, 0.f}, false);
+    DecArgs a{dst, nullptr, q, kc, vc, nullptr, nullptr, kv_len, hd, n_heads, n_kv_heads, 0, 0.f};
+    const size_t bytes = attention_decode_part_bytes(kv_len, hd, n_heads);
+    if (bytes) {
+        const StreamScratch scratch(bytes);
+        a.part = (float *)scratch.get();
+        decode_attention(a, false);
+    } else {
+        decode_attention(a, false);
+    }
 }
 
 void attention_decode_rope(float *dst, const float *q, const float *kx, float *kc, const float *vc, int pos, int hd,
-                           int n_heads, int n_kv_heads, float base)
+                           int n_heads, int n_kv_heads, float base, float *part)
 {
-    decode_attention(DecArgs{dst, nullptr, q, kc, vc, kx, kc + (int64_t)pos * n_kv_heads * hd, pos + 1, hd, n_heads,
+    decode_attention(DecArgs{dst, part, q, kc, vc, kx, kc + (int64_t)pos * n_kv_heads * hd, pos + 1, hd, n_heads,
                              n_kv_heads, 0, base},
                      true);
-}
-
-bool attention_scratch_init()
-{
-    if (g_dec_part) return true;
-    if (hipMalloc((void **)&g_dec_part, kDecPartFloats * sizeof(float)) != hipSuccess) {
-        g_dec_part = nullptr;
-        return false;
-    }
-    return true;
-}
-
-void attention_scratch_release()
-{
-    if (g_dec_part) (void)hipFree(g_dec_part);
-    g_dec_part = nullptr;
 }
 
 // ---- RoPE (cuda_ops.cu:2102-2140): pairs (i, i + hd/2), theta = pos / base^(2i/hd) ----------

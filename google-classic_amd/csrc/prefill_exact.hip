@@ -1506,7 +1506,6 @@ void q6r_repack(void *out, const void *W, int N, int K)
 
 void exact_release()
 {
-    few_rows_release();
     if (g_x2_cnt) (void)hipFree(g_x2_cnt);
     g_x2_cnt = nullptr;
     prepared_release_all();

@@ -6,8 +6,10 @@
 #include <atomic>
 #include <mutex>
 #include <string.h>
+#include <unordered_map>
 
 #include "common.h"
+#include "stream_scratch.h"
 
 namespace {
 
@@ -17,6 +19,8 @@ hipStream_t g_stream = nullptr;       // library compute stream (null = legacy d
 hipStream_t g_copy_stream = nullptr;  // cuda_memcpy_*_async
 int g_cus = 256;
 std::atomic<int> g_error{0};
+std::mutex g_graph_mu;
+std::unordered_map<hipGraphExec_t, unsigned long long> g_graph_capture;  // its capture's id
 
 }  // namespace
 
@@ -103,8 +107,8 @@ int cuda_init(void)
         fprintf(stderr, "holo_mi355x: cannot allocate the GEMV stream barrier\n");
         return -1;
     }
-    if (!holo::attention_scratch_init()) {
-        fprintf(stderr, "holo_mi355x: cannot allocate the decode-attention scratch\n");
+    if (!holo::stream_scratch_init()) {
+        fprintf(stderr, "holo_mi355x: cannot allocate the captured calls' scratch\n");
         return -1;
     }
     if (!holo::exact_init()) {
@@ -127,7 +131,7 @@ void cuda_cleanup(void)
     if (g_copy_stream) hipStreamDestroy(g_copy_stream);
     g_copy_stream = nullptr;
     holo::gemv_stream_release();
-    holo::attention_scratch_release();
+    holo::stream_scratch_release();
     holo::panel_workspace_release();
     holo::exact_release();
     g_stream = nullptr;
@@ -249,7 +253,7 @@ void *holo_stream_create(void)
 void holo_stream_destroy(void *s)
 {
     if (!s) return;
-    holo::few_rows_drop_stream((hipStream_t)s);
+    holo::stream_scratch_drop((hipStream_t)s);
     HOLO_CHECK(hipStreamDestroy((hipStream_t)s));
 }
 
@@ -293,17 +297,24 @@ void *holo_graph_end(void)
 {
     hipGraph_t g = nullptr;
     hipGraphExec_t ge = nullptr;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    (void)hipStreamGetCaptureInfo(g_stream, &st, &id);
     hipError_t e = hipStreamEndCapture(g_stream, &g);
     if (e != hipSuccess) {
+        holo::stream_scratch_drop_capture(id);
         holo::latch_error((int)e, "hipStreamEndCapture", __FILE__, __LINE__);
         return nullptr;
     }
     e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) {
+        holo::stream_scratch_drop_capture(id);
         holo::latch_error((int)e, "hipGraphInstantiate", __FILE__, __LINE__);
         return nullptr;
     }
+    std::lock_guard<std::mutex> lk(g_graph_mu);
+    g_graph_capture[ge] = id;
     return (void *)ge;
 }
 
@@ -319,7 +330,18 @@ int holo_graph_launch(void *graph_exec)
 
 void holo_graph_destroy(void *graph_exec)
 {
-    if (graph_exec) HOLO_CHECK(hipGraphExecDestroy((hipGraphExec_t)graph_exec));
+    if (!graph_exec) return;
+    unsigned long long id = 0;
+    {
+        std::lock_guard<std::mutex> lk(g_graph_mu);
+        const auto it = g_graph_capture.find((hipGraphExec_t)graph_exec);
+        if (it != g_graph_capture.end()) {
+            id = it->second;
+            g_graph_capture.erase(it);
+        }
+    }
+    HOLO_CHECK(hipGraphExecDestroy((hipGraphExec_t)graph_exec));
+    if (id) holo::stream_scratch_drop_capture(id);
 }
 
 }  // extern "C"

@@ -128,3 +128,90 @@ def test_decode_very_low_scores(holo, synth, hd, nh, nkv, kv_len, first, low):
     # equal weights are exact, so only the sums of values round: their terms
     # are N(0, 1), their mean N(0, 1) / sqrt(n)
     assert np.max(np.abs(down(d, nh * hd) - want)) <= 8 * 2.0**-24
+
+
+@pytest.mark.parametrize("kv_len", [600, 3000])
+def test_decode_streams_and_graph(holo, synth, kv_len):
+    """Calls of several ranges under way on two streams at once, and a captured
+    graph replayed beside them: the bits of each call on its own."""
+    print(f"case decode streams kv_len {kv_len}", flush=True)
+    lib = holo.lib()
+    hd, nh, nkv = 128, 32, 8
+    kc, vc = (up(holo, synth.normal(kv_len * nkv * hd, seed=90 + i)) for i in range(2))
+    qs = [up(holo, synth.normal(nh * hd, seed=s)) for s in (92, 93)]
+
+    def call(q):
+        d = holo.DeviceBuffer(4 * nh * hd)
+        lib.cuda_multi_head_attention(d.ptr, q.ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+        return d
+
+    want = [call(q) for q in qs]
+    lib.cuda_sync()
+    want = [down(d, nh * hd).view(np.uint32) for d in want]
+    streams = [lib.holo_stream_create() for _ in range(2)]
+    try:
+        got = []
+        for _ in range(20):
+            for s, q in zip(streams, qs):
+                lib.holo_set_stream(s)
+                got.append(call(q))
+        lib.cuda_sync()
+        for i, d in enumerate(got):
+            assert np.array_equal(down(d, nh * hd).view(np.uint32), want[i % 2]), i
+        dG = holo.DeviceBuffer(4 * nh * hd)
+        lib.holo_set_stream(streams[0])
+        assert lib.holo_graph_begin() == 0
+        for _ in range(8):
+            lib.cuda_multi_head_attention(dG.ptr, qs[0].ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+        g = lib.holo_graph_end()
+        holo.check("capture")
+        for rep in range(4):
+            lib.holo_set_stream(streams[0])
+            lib.holo_graph_launch(g)
+            lib.holo_set_stream(streams[1])
+            beside = [call(qs[1]) for _ in range(8)]
+            lib.cuda_sync()
+            assert np.array_equal(down(dG, nh * hd).view(np.uint32), want[0]), rep
+            for d in beside:
+                assert np.array_equal(down(d, nh * hd).view(np.uint32), want[1]), rep
+        lib.holo_graph_destroy(g)
+    finally:
+        lib.holo_set_stream(None)
+        for s in streams:
+            lib.holo_stream_destroy(s)
+    holo.check("streams")
+
+
+def test_decode_graphs_own_their_partials(holo, synth):
+    """More captured graphs alive than the library's capture scratch holds, and
+    again after they are gone: every replay gives the eager call's bits."""
+    lib = holo.lib()
+    hd, nh, nkv, kv_len = 128, 32, 8, 600
+    kc, vc = (up(holo, synth.normal(kv_len * nkv * hd, seed=94 + i)) for i in range(2))
+    qs = [up(holo, synth.normal(nh * hd, seed=96 + i)) for i in range(4)]
+    want = []
+    for q in qs:
+        d = holo.DeviceBuffer(4 * nh * hd)
+        lib.cuda_multi_head_attention(d.ptr, q.ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+        want.append(down(d, nh * hd).view(np.uint32))
+    s = lib.holo_stream_create()
+    lib.holo_set_stream(s)
+    try:
+        for turn in range(2):
+            graphs = []
+            for i in range(130):  # 16 MiB in parts of 132 KiB
+                d = holo.DeviceBuffer(4 * nh * hd)
+                assert lib.holo_graph_begin() == 0
+                lib.cuda_multi_head_attention(d.ptr, qs[i % 4].ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+                graphs.append((lib.holo_graph_end(), d))
+            holo.check("captures")
+            for g, _ in graphs:
+                lib.holo_graph_launch(g)
+            lib.cuda_sync()
+            for i, (g, d) in enumerate(graphs):
+                assert np.array_equal(down(d, nh * hd).view(np.uint32), want[i % 4]), (turn, i)
+                lib.holo_graph_destroy(g)
+    finally:
+        lib.holo_set_stream(None)
+        lib.holo_stream_destroy(s)
+    holo.check("graphs")
