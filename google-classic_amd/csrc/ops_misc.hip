@@ -890,15 +890,16 @@ __global__ __launch_bounds__(128) void attn_dec_merge_k(float *out, const float 
 #pragma unroll
         for (int s = 1; s < NS; s++) mx = fmaxf(mx, m[s]);
         const float c = __builtin_amdgcn_exp2f(M - mx);  // 0 in the first round
-        L *= c;
-        a *= c;
         M = mx;
+        float Ls[4] = {}, as[4] = {};  // four short sums round less than one long one
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const float w = __builtin_amdgcn_exp2f(m[s] - M);
-            L = fmaf(w, l[s], L);
-            a = fmaf(w, o[s], a);
+            Ls[s & 3] = fmaf(w, l[s], Ls[s & 3]);
+            as[s & 3] = fmaf(w, o[s], as[s & 3]);
         }
+        L = fmaf(L, c, (Ls[0] + Ls[1]) + (Ls[2] + Ls[3]));
+        a = fmaf(a, c, (as[0] + as[1]) + (as[2] + as[3]));
     }
     if (d < hd) out[(int64_t)h * hd + d] = a * (1.0f / L);
 }
@@ -1012,15 +1013,20 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
         }
         const float corr = __builtin_amdgcn_exp2f(m - mx);
         m = mx;
-        l *= corr;
-        o4 = make_float4(o4.x * corr, o4.y * corr, o4.z * corr, o4.w * corr);
+        // the pass's keys are summed first: one rounding a pass at the size of
+        // the sums so far instead of five (with the merges in four short sums,
+        // 4096 positions of 32 heads are 1.84e-7 off in 2-norm, else 2.05e-7)
+        float ls = 0.f;
+        float4 os = zero;
 #pragma unroll
         for (int j = 0; j < J; j++) {
             const float w = __builtin_amdgcn_exp2f(sj[j] - m);
-            l += w;
-            o4 = make_float4(fmaf(w, v4[b][j].x, o4.x), fmaf(w, v4[b][j].y, o4.y), fmaf(w, v4[b][j].z, o4.z),
-                             fmaf(w, v4[b][j].w, o4.w));
+            ls += w;
+            os = make_float4(fmaf(w, v4[b][j].x, os.x), fmaf(w, v4[b][j].y, os.y), fmaf(w, v4[b][j].z, os.z),
+                             fmaf(w, v4[b][j].w, os.w));
         }
+        l = fmaf(l, corr, ls);
+        o4 = make_float4(fmaf(o4.x, corr, os.x), fmaf(o4.y, corr, os.y), fmaf(o4.z, corr, os.z), fmaf(o4.w, corr, os.w));
     };
     for (int p0 = p_begin; p0 < p_end; p0 += 2 * G * J) {
         use(0, p0);
@@ -1050,13 +1056,14 @@ __global__ __launch_bounds__(kDecThreads) void attn_dec_k(DecArgs a)
         float M = lm[0];
 #pragma unroll
         for (int w = 1; w < W; w++) M = fmaxf(M, lm[w]);
-        float L = 0.f, r = 0.f;
+        float Ls[4] = {}, rs[4] = {};
 #pragma unroll
         for (int w = 0; w < W; w++) {
             const float e = __builtin_amdgcn_exp2f(lm[w] - M);
-            L = fmaf(e, ll[w], L);
-            r = fmaf(e, lo[w][t], r);
+            Ls[w & 3] = fmaf(e, ll[w], Ls[w & 3]);
+            rs[w & 3] = fmaf(e, lo[w][t], rs[w & 3]);
         }
+        const float L = (Ls[0] + Ls[1]) + (Ls[2] + Ls[3]), r = (rs[0] + rs[1]) + (rs[2] + rs[3]);
         if (splits == 1) {
             a.out[(int64_t)h * hd + t] = r * (1.0f / L);
         } else {
