@@ -4,6 +4,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+// Between LDS accesses through which the lanes of one wave hand data to each
+// other.  The hardware keeps a wave's LDS accesses in order; this keeps the
+// compiler from moving one past another that is of another address or type.
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 __device__ __forceinline__ float wave_reduce_sum(float v)
 {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

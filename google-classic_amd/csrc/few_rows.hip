@@ -510,7 +510,7 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
     const int pl = min(lane, U::RI * U::NP - 1), pr = pl / U::NP, pc = pl - pr * U::NP;
     const uint32_t row0 = (uint32_t)(nl + (ST ? pr : (int)c)) * rowb + mis;
     const uint32_t wo = row0 + (ST ? 16u * (uint32_t)pc : 0u);
-    uint8_t *const put = stage + pr * U::STRIDE + 16 * pc;
+    uint32_t put = (uint32_t)(pr * U::STRIDE + 16 * pc);  // in the stage
     const uint8_t *const get = stage + c * U::STRIDE;
     // byte phase of the lane's windows (Q6_K: of its column's row, the unit's comes on top)
     const uint32_t phase = WF == EW_Q6_K ? ((uint32_t)(nl + (int)c) * rowb + mis) & 2u
@@ -540,8 +540,13 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
         }
     };
     auto stash_unit = [&]() {
+        // what one lane stores others read: with an offset that the compiler does
+        // not know it cannot move a read past these stores, nor the next ones past
+        // a read (wave_lds_fence, which holds back the loads of the next unit too,
+        // makes 16 x 11008 x 4096 take 16.0 us instead of 14.9)
+        asm("" : "+v"(put));
 #pragma unroll
-        for (int i = 0; i < NI; i++) *(v4u *)(put + U::RI * i * U::STRIDE) = wr[i];
+        for (int i = 0; i < NI; i++) *(v4u *)(stage + put + U::RI * i * U::STRIDE) = wr[i];
     };
     auto fetch_raw = [&](int u, int e) {
         const __amdgpu_buffer_rsrc_t r = wrsrc(u);

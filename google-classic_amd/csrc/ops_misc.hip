@@ -389,10 +389,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_mfma_k(float *ou
 #pragma unroll
         for (int c = 0; c < NQ; c++) {
             if (c % (DH / 16) == 0) {
-                // this wave's own stage: its LDS accesses stay in order, so the
-                // reads below need no barrier, nor these writes after the last ones
+                // this wave's own stage: neither the reads below nor these writes
+                // after the last ones need a barrier
+                wave_lds_fence();
 #pragma unroll
                 for (int i = 0; i < NI; i++) *(float4 *)(kput + RPI * i * KS) = kr[c / (DH / 16)][i];
+                wave_lds_fence();
             }
             const float4 ka = *(const float4 *)(kget + 16 * (c % (DH / 16)));
             const float4 kb = *(const float4 *)(kget + 16 * (c % (DH / 16)) + 4);
@@ -753,6 +755,7 @@ __global__ __launch_bounds__(64 * kQ6Waves) void gemv_q6_k3_k(float *dst, const 
     for (int rr = 0; rr < R; rr++) acc[rr] = 0.f;
     while (grp < ngroup) {
         uint32_t ph[R];
+        wave_lds_fence();
 #pragma unroll
         for (int rr = 0; rr < R; rr++) {
             ph[rr] = (uint32_t)(((uintptr_t)M + (int64_t)min(grp * R + rr, out - 1) * row_bytes + (int64_t)pass * kQ6Run) & 15u);
@@ -761,6 +764,7 @@ __global__ __launch_bounds__(64 * kQ6Waves) void gemv_q6_k3_k(float *dst, const 
                 if (64 * (i + 1) <= kQ6Pieces || lane + 64 * i < kQ6Pieces)
                     *(uint4 *)(stage + rr * kQ6Stage + 16 * (lane + 64 * i)) = pw[rr][i];
         }
+        wave_lds_fence();
         const bool done = pass + 1 == npass;  // of this group
         const int ng = done ? grp + step : grp, np = done ? 0 : pass + 1;
         fetch(ng, np);
