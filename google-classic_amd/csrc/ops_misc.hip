@@ -826,17 +826,23 @@ __global__ __launch_bounds__(64 * kQ6Waves) void gemv_q6_k3_k(float *dst, const 
     }
 }
 
-// Rows per wave: the most (of 4, 2, 1) that still give two workgroups per CU
-// (MI355X: 4 rows at 32000 and 11008 rows, 2 at 4096).  HOLO_Q6K_ROWS=1|2|4
-// forces a value.
-static int q6_rows_per_wave(int out_dim)
+// HOLO_Q6K_ROWS=1|2|4: straight loads with that many rows per wave, at any row
+// count (0: not set).
+static int q6_forced_rows()
 {
     static const int forced = [] {
         const char *e = getenv("HOLO_Q6K_ROWS");
         const int v = e ? atoi(e) : 0;
         return (v == 1 || v == 2 || v == 4) ? v : 0;
     }();
-    if (forced) return forced;
+    return forced;
+}
+
+// Rows per wave: the most (of 4, 2, 1) that still give two workgroups per CU
+// (MI355X: 4 rows at 11008 rows, 2 at 4096).
+static int q6_rows_per_wave(int out_dim)
+{
+    if (q6_forced_rows()) return q6_forced_rows();
     for (int r = 4; r > 1; r /= 2)
         if ((out_dim + 4 * r - 1) / (4 * r) >= 2 * num_cus()) return r;
     return 1;
@@ -1839,7 +1845,8 @@ void cuda_matmul_q6_k(float *dst, const void *M, const float *v, int out_dim, in
     // modes keep fp32 activations.
     const size_t lds = (size_t)(in_dim / 256) * 1024 + (size_t)kQ6Waves * kQ6Rows * kQ6Stage;
     const int wgs = (lds <= 80 * 1024 ? 2 : 1) * num_cus();
-    if (lds <= 160 * 1024 && out_dim >= 2 * kQ6Rows * kQ6Waves * wgs && gemv_default_mode()) {
+    if (lds <= 160 * 1024 && out_dim >= 2 * kQ6Rows * kQ6Waves * wgs && gemv_default_mode() &&
+        !q6_forced_rows()) {
         static const hipError_t attr = hipFuncSetAttribute((const void *)gemv_q6_k3_k,
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (attr != hipSuccess) {

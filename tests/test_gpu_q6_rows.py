@@ -8,6 +8,11 @@ largest magnitude a each, its sum, scale and product round five times, a lane
 adds 4 groups a pass and the wave's tree 6 more: (4 passes + 16) 2^-24 sum over
 groups a_g sum |w|.
 """
+import os
+import pathlib
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -53,3 +58,29 @@ def test_q6_many_rows(holo, synth, oracle, rows, K, off):
         print(f"  {case}: max err / bound {np.max(err / bound):.3f}", flush=True)
         assert np.all(err <= bound), case
         assert np.array_equal(got[:rows], np.concatenate([got[:n]] * (rows // n + 1))[:rows])
+
+
+def test_q6_forced_rows(holo, synth, oracle):
+    """HOLO_Q6K_ROWS keeps straight loads at any row count: the bits of a call
+    of few rows.  (It is read once a process, so in one of its own.)"""
+    code = """
+import sys
+sys.path[:0] = ["google-classic_amd", "tests", "."]
+import numpy as np, holo_mi355x as holo
+from holo_mi355x import synth
+holo.load(); holo.init()
+lib = holo.lib()
+raw = np.frombuffer(np.ascontiguousarray(synth.blocks(14, 100, 4096, 5)).tobytes(), np.uint8)
+w = holo.DeviceBuffer.from_array(np.tile(raw, 165))
+x = holo.DeviceBuffer.from_array(synth.normal(4096, seed=6))
+a, b = holo.DeviceBuffer(400), holo.DeviceBuffer(4 * 16500)
+lib.cuda_matmul_q6_k(a.ptr, w.ptr, x.ptr, 100, 4096)
+lib.cuda_matmul_q6_k(b.ptr, w.ptr, x.ptr, 16500, 4096)
+lib.cuda_sync()
+holo.check("forced rows")
+assert np.array_equal(np.tile(a.download(np.float32, 100), 165), b.download(np.float32, 16500))
+"""
+    root = pathlib.Path(__file__).resolve().parent.parent
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, env={**os.environ, "HOLO_Q6K_ROWS": "2"}, timeout=60,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
