@@ -1,7 +1,9 @@
 """cuda_matmul_q6_k with enough rows for the staged kernel: an odd row count,
-one and two passes of 16 superblocks a row (whole and partial), the largest
-staged row and the first past it, matrices off 4- and 16-byte alignment, and
-activations that are tiny, zero in places or not finite.
+one and two passes of 16 superblocks a row (whole and partial), long rows, the
+longest staged one (27392: 160 KiB of LDS) and the first past it, matrices off
+4- and 16-byte alignment, and activations that are tiny, zero in places, not
+finite (NaN, as from the straight kernel, whose 32 sum(x) meets sum(q x)) or
+with outliers.
 
 Bar, from the number formats: a group of 16 activations is within 2^-24 of its
 largest magnitude a each, its sum, scale and product round five times, a lane
@@ -20,7 +22,8 @@ from test_gpu_batch_exact import Q6_K, down, up, weights
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(16385, 256, 0), (16384, 4096, 2), (17001, 4352, 14), (16390, 768, 6), (8193, 24576, 0), (8193, 26624, 2)]
+CASES = [(16385, 256, 0), (16384, 4096, 2), (17001, 4352, 14), (16390, 768, 6), (8193, 24576, 0), (8193, 26624, 2),
+         (8193, 27392, 0), (8193, 27392, 6), (8193, 27648, 2)]
 
 
 @pytest.mark.parametrize("rows,K,off", CASES)
@@ -58,6 +61,43 @@ def test_q6_many_rows(holo, synth, oracle, rows, K, off):
         print(f"  {case}: max err / bound {np.max(err / bound):.3f}", flush=True)
         assert np.all(err <= bound), case
         assert np.array_equal(got[:rows], np.concatenate([got[:n]] * (rows // n + 1))[:rows])
+
+
+@pytest.mark.parametrize("ratio", [1.0, 30.0, 1e3, 1e6])
+def test_q6_outliers(holo, synth, oracle, ratio):
+    """An outlier in every group of 16, facing weights of zero (q = 32): the
+    outliers' rounding is all that shows, in the staged kernel (a group's fixed
+    point) as in the straight one (sum(q x) - 32 sum(x)).  The staged kernel's
+    error against 64 bits (2-norm) stays within 1.2 of the straight one's, and
+    below it without outliers."""
+    print(f"case q6 outliers {ratio}", flush=True)
+    lib = holo.lib()
+    n, rows, K = 500, 16400, 4096
+    src, _ = weights(synth, oracle, Q6_K, n, K, seed=77)
+    raw = np.frombuffer(np.ascontiguousarray(src).tobytes(), np.uint8).reshape(n, K // 256, 210).copy()
+    x = synth.normal(K, seed=78)
+    if ratio > 1:
+        for i in range(0, K, 16):
+            i += (7 * i // 16) % 16
+            x[i] *= np.float32(ratio)
+            b, r = divmod(i, 256)
+            h, r = divmod(r, 128)
+            j, l = divmod(r, 32)
+            low, high = 64 * h + 32 * (j & 1) + l, 128 + 32 * h + l
+            raw[:, b, low] &= 0x0F if j >> 1 else 0xF0
+            raw[:, b, high] = raw[:, b, high] & ~np.uint8(3 << 2 * j) | np.uint8(2 << 2 * j)
+    w = np.asarray(oracle.dequant(Q6_K, raw.reshape(-1), n * K), np.float64).reshape(n, K)
+    many = np.concatenate([raw.reshape(n, -1)] * (rows // n + 1))[:rows].reshape(-1)
+    dM, dx = up(holo, many), up(holo, x)
+    ds, dm = holo.DeviceBuffer(4 * n), holo.DeviceBuffer(4 * rows)
+    lib.cuda_matmul_q6_k(ds.ptr, dM.ptr, dx.ptr, n, K)
+    lib.cuda_matmul_q6_k(dm.ptr, dM.ptr, dx.ptr, rows, K)
+    lib.cuda_sync()
+    holo.check("q6 outliers")
+    truth = w @ x.astype(np.float64)
+    straight, staged = (np.linalg.norm(down(d, n) - truth) / np.linalg.norm(truth) for d in (ds, dm))
+    print(f"  straight {straight:.2e}, staged {staged:.2e}", flush=True)
+    assert staged <= (1.2 if ratio > 1 else 1.0) * straight
 
 
 def test_q6_forced_rows(holo, synth, oracle):
