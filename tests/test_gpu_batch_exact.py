@@ -1,6 +1,10 @@
 """GPU parity of the exact batched product (HOLO_PREFILL_EXACT, the default of
 holo_matmul_batch* and of the prompt forward), through the C ABI.
 
+Many shapes here run the tiles for few rows (few_rows.hip; up to 1024 rows where
+they are the faster ones): every such tile is in test_gpu_few_rows_plans, ragged
+shapes on the 64 x 256 tiles in test_gpu_exact_tiles.
+
 The product (prefill_exact.hip) holds the activations as two f16 halves
 (x = xh + xl to 2^-22), the weights as the blocks' exact integers with
 their fp32 scales, and accumulates in fp32.  Its truth is the float64 product
@@ -309,9 +313,9 @@ def test_prepared_q6_k(holo, synth, oracle, M, N, K):
 
 
 def _sweep_shapes():
-    """Seeded small shapes per type: M from 64 (the batched path's least) to
-    ragged row tiles, N ragged against the 32-, 64- and 256-column tiles, K
-    from one block (one superblock for Q4_K/Q6_K) to a few hundred."""
+    """Seeded small shapes per type: M from 64 to ragged row tiles, N ragged
+    against 16- to 64-column tiles, K from one block (one superblock for
+    Q4_K/Q6_K) to a few hundred.  All run the tiles for few rows."""
     rng = np.random.default_rng(2024)
     out = []
     for t in (Q4_0, Q8_0, Q4_K, Q6_K, F16):
@@ -362,7 +366,8 @@ def test_exact_part_shapes(holo, synth, oracle, t, M, N, K):
     accumulators) or stores its part and counts; the 4096-wide o/v shape, whose
     parts are mapped to XCDs; a last column tile 64 wide (2112).  Two calls
     give the same bits, and the first and last row of every 32-row band are
-    within the bound of the float64 truth."""
+    within the bound of the float64 truth.  (192 x 11008 and 320 x 2112 run
+    the tiles for few rows.)"""
     print(f"case exact parts {NAMES[t]} {M}x{N}x{K}", flush=True)
     lib = holo.lib()
     src, w = weights(synth, oracle, t, N, K, seed=3 * M + N + K)

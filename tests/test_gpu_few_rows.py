@@ -16,10 +16,10 @@ from test_gpu_batch_exact import F16, NAMES, Q4_0, Q4_K, Q6_K, Q8_0, check_rows,
 
 pytestmark = pytest.mark.gpu
 
-# rows at the edges of 16-row tiles and of the 1, 2 and 4 tiles a workgroup
-# takes; columns at the edges of 16- to 64-column tiles; K of one block, odd
-# block counts (windows straight from memory), one unit of 256, more units
-# than waves, and K split over several workgroups
+# rows at the edges of 16- and 64-row tiles; columns at the edges of 16- and
+# 32-column tiles; K of one block, odd block counts (windows straight from
+# memory), one unit of 256, more units than waves, and K split over several
+# workgroups (every tile that can run: test_gpu_few_rows_plans)
 CASES = [(Q4_0, 3, 1, 32), (Q4_0, 16, 15, 256), (Q4_0, 17, 16, 288), (Q4_0, 33, 301, 1056), (Q4_0, 64, 4096, 4096),
          (Q4_0, 20, 1000, 11008), (Q4_0, 130, 100, 2304), (Q4_0, 192, 333, 1024), (Q8_0, 3, 17, 32),
          (Q8_0, 15, 49, 2080), (Q8_0, 32, 130, 4096), (Q8_0, 63, 64, 544), (Q8_0, 50, 700, 8192), (Q4_K, 4, 3, 256),
