@@ -28,10 +28,10 @@ namespace holo {
 // cannot hold a row with infinities (an infinity's low half is a NaN, its
 // block sum meets the min term's infinity, its neighbours have no common
 // scale), nor, in full, one with a 32-block that lies wholly below a * 2^-17
-// (where the low half runs out of f16's exponents): such a row leaves its fp32
-// values in the place of its operands, and Rs = -1 tells the product to take it
-// from them.  Small blocks count only with `range`: the GEMVs, which few rows
-// would take otherwise, scale every block by itself, the other tiles do not.
+// (where the low half runs out of f16's exponents): such a row's fp32 values go
+// to X32 [M][K], and Rs = -1 tells the product to take it from there.  Small
+// blocks count only with `range`: the GEMVs, which few rows would take
+// otherwise, scale every block by itself, the other tiles do not.
 // PART (with OPS): gridDim.y workgroups share a row: each finds the row's
 // scale from all of it and splits and stores float4s part * blockIdx.y ..
 // of it (part a multiple of 8 and at most NT), which it loads a second time.
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
                                                     float *__restrict__ Sx, float *__restrict__ Rs,
                                                     const float *__restrict__ X, const float *__restrict__ U,
                                                     const float *__restrict__ NW, int K, float eps, uint32_t *zero,
-                                                    int n_zero, int part, bool range)
+                                                    int n_zero, int part, bool range, float *X32)
 {
     static_assert(OPS || !PART);
     __shared__ float red[16];
@@ -238,8 +238,8 @@ __global__ __launch_bounds__(NT) void xsplit_row_k(uint2 *__restrict__ Ah, uint2
             if (PART ? mine : i < n4) {
                 const int64_t b = (int64_t)(blockIdx.x >> 4) * (n4 >> 3) + (i >> 3);
                 const int m = blockIdx.x & 15;
-                ((uint4 *)Ah)[b * 128 + m + 16 * (i & 3) + (up ? 64 : 0)] =
-                    raw ? __builtin_bit_cast(uint4, x) : up ? make_uint4(t0, t1, l0, l1) : make_uint4(h0, h1, t0, t1);
+                if (raw) ((float4 *)X32)[r4 + i] = x;
+                ((uint4 *)Ah)[b * 128 + m + 16 * (i & 3) + (up ? 64 : 0)] = up ? make_uint4(t0, t1, l0, l1) : make_uint4(h0, h1, t0, t1);
                 if (Sx && (i & 7) == 0) Sx[b * 16 + m] = s;
             }
         } else if (i < n4) {

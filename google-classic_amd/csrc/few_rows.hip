@@ -66,7 +66,8 @@ struct FrArgs {
     int t_end[kExactMats];  // prefix sums of their column tiles; unused entries INT_MAX
     const uint8_t *A;       // activation halves in operand order
     const float *Sx;        // [M/16][nb][16] block sums (Q4_K)
-    const float *Rs;        // [M] row scales
+    const float *Rs;        // [M] row scales; -1: the row is in X32 instead
+    const float *X32;       // [M][32 nb] fp32 values of such rows
     const float *R;         // one matrix only: Y = R + product (may alias Y)
     float *part;
     uint32_t *cnt;
@@ -442,21 +443,34 @@ __device__ __forceinline__ float4 fr_weights(const uint8_t *row, int b, int i)
                        d * ((float)((q >> 16) & 255u) - off) - mn, d * ((float)(q >> 24) - off) - mn);
 }
 
-// Row m of the activations, left as fp32 values in the place of its operands
-// (xsplit_row_k), times a weight row: a wave, lane l blocks l, l + 64, ...
+// fp32 activation rows (those of the four from x on that `rows` has a bit for)
+// times a weight row, by a wave: consecutive lanes take consecutive weights,
+// every lane gets the sums.
 template <int WF>
-__device__ __forceinline__ float fr_dot(const uint8_t *row, const uint8_t *A, int m, int nb, int lane)
+__device__ __forceinline__ float4 fr_dot4(const uint8_t *row, const float *x, uint32_t rows, int nb, int lane)
 {
-    float s = 0.f;
-    for (int b = lane; b < nb; b += 64) {
-        const float4 *x = (const float4 *)(A + ((int64_t)(m >> 4) * nb + b) * 2048) + (m & 15);
-#pragma unroll 1
-        for (int i = 0; i < 8; i++) {
-            const float4 v = x[16 * (i & 3) + 64 * (i >> 2)], w = fr_weights<WF>(row, b, i);
-            s = fmaf(w.w, v.w, fmaf(w.z, v.z, fmaf(w.y, v.y, fmaf(w.x, v.x, s))));
+    const float4 *x4 = (const float4 *)x;
+    const int n4 = 8 * nb;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = lane; k0 < n4; k0 += 256) {
+        float4 w[4], v[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int k = min(k0 + 64 * u, n4 - 1);
+            w[u] = fr_weights<WF>(row, k >> 3, k & 7);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if ((rows >> r) & 1u) v[u][r] = x4[(int64_t)r * n4 + k];
         }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k0 + 64 * u < n4)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if ((rows >> r) & 1u)
+                        s[r] = fmaf(w[u].w, v[u][r].w, fmaf(w[u].z, v[u][r].z, fmaf(w[u].y, v[u][r].y, fmaf(w[u].x, v[u][r].x, s[r]))));
     }
-    return wave_reduce_sum(s);
+    return make_float4(wave_reduce_sum(s[0]), wave_reduce_sum(s[1]), wave_reduce_sum(s[2]), wave_reduce_sum(s[3]));
 }
 
 __device__ __forceinline__ v4f mfma_k32(v4u a, v4u b, v4f c)
@@ -582,6 +596,7 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
     v4u av[2][GB][MT][2];
     float sx[2][MT];
 
+    const float row_scale = a.Rs[min(rt0 * 16 + lane, a.M - 1)];  // here, so that its wait is over at the end
     load_a(av[0], 8 * u0);
     load_sx(sx[0], 2 * u0);
     if constexpr (ST) {
@@ -672,6 +687,8 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
             }
         }
     }
+    // the workgroup's rows whose fp32 values were left: bit i, row i
+    const uint64_t whole = __ballot(lane < 16 * MT && rt0 * 16 + lane < a.M && row_scale < 0.f);
     if constexpr (ST) __syncthreads();  // the sums' buffer lies over the stages
 
     // the waves' sums, in wave order
@@ -745,24 +762,27 @@ __global__ __launch_bounds__(64 * kFrWaves, 1) void gemm_few_k(FrArgs a)
             rs[r] = a.Rs[m];
             rv[r] = a.R ? a.R[(int64_t)m * Nm + min(n, Nm - 1)] : 0.f;
         }
-        bool raw = false;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            raw = raw || (m0 + r < a.M && n < Nm && rs[r] < 0.f);
+        for (int r = 0; r < 4; r++)
             if (m0 + r < a.M && n < Nm && !(rs[r] < 0.f)) {
                 const float y = v[i][r] * rs[r];  // a power of two: exact
                 Ym[(int64_t)(m0 + r) * Nm + n] = a.R ? rv[r] + y : y;
             }
-        }
-        // rows that the halves do not hold: fp32 products, an output at a time
-        for (uint64_t todo = __ballot(raw); todo; todo &= todo - 1) {
-            const int l = __builtin_ctzll(todo), nn = nl + 16 * (t % CT) + (l & 15);
-            for (int r = 0; r < 4; r++) {
-                const int m = (rt0 + t / CT) * 16 + 4 * (l >> 4) + r;
-                if (m >= a.M || !(a.Rs[m] < 0.f)) continue;
-                const float y = fr_dot<WF>(Wm + (int64_t)nn * rowb, a.A, m, nb, lane);
-                const int64_t at = (int64_t)m * Nm + nn;
-                if (lane == 0) Ym[at] = a.R ? a.R[at] + y : y;
+    }
+    // rows that the halves do not hold: fp32 products, each wave columns of its
+    // own, four rows at a time (16 x 11008 x 4096 Q4_0 with 0, 1 and 16 such rows
+    // 14.2, 38.6 and 139 us; a GEMV per row 114; the values read back from operand
+    // order, in 16-byte pieces, 105 and 370)
+    for (int q = 0; whole != 0 && q < 4 * MT; q++) {
+        const uint32_t rows = (uint32_t)(whole >> (4 * q)) & 15u;
+        if (rows == 0) continue;
+        for (int c16 = wave; c16 < 16 * CT && nl + c16 < Nm; c16 += kFrWaves) {
+            const int m = rt0 * 16 + 4 * q;
+            const float4 y = fr_dot4<WF>(Wm + (int64_t)(nl + c16) * rowb, a.X32 + (int64_t)m * 32 * nb, rows, nb, lane);
+            const int64_t at = (int64_t)(m + lane) * Nm + nl + c16;
+            if (lane < 4 && (rows >> lane) & 1u) {
+                const float v1 = lane == 0 ? y.x : lane == 1 ? y.y : lane == 2 ? y.z : y.w;
+                Ym[at] = a.R ? a.R[at] + v1 : v1;
             }
         }
     }
@@ -973,13 +993,15 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t ob = up((size_t)ntm * nb * 2048), sb = c.need_sx ? up((size_t)ntm * nb * 64) : 0, rb = up((size_t)M * 4),
                  cb = up((size_t)counters * 4);
-    const size_t total = ob + sb + rb + cb + parts;
+    const size_t xb = up((size_t)M * K * 4);
+    const size_t total = ob + sb + rb + cb + xb + parts;
     const StreamScratch scratch(total);
     uint8_t *ws = (uint8_t *)scratch.get();
     if (!ws) return false;
     uint8_t *A = ws;
     float *Sx = c.need_sx ? (float *)(ws + ob) : nullptr, *Rs = (float *)(ws + ob + sb);
     uint32_t *cnt = (uint32_t *)(ws + ob + sb + rb);
+    float *X32 = (float *)(ws + ob + sb + rb + cb);
     // Few rows leave most CUs idle: four workgroups a row (each of at most
     // `most` float4s) while they fit the CUs.  23 rows, alone -> four -> eight:
     // SwiGLU 11008 wide 8.6 -> 6.6 -> 7.5 us, the norm 4096 wide 5.0 -> 4.6 ->
@@ -994,7 +1016,7 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
     };
     auto split = [&](auto kern, int nt) {
         hipLaunchKernelGGL(kern, dim3(M, shares), dim3(nt), 0, stream(), (uint2 *)A, (uint2 *)nullptr, Sx, Rs, X, U, NW, K,
-                           eps, cnt, counters, part, M < 64);
+                           eps, cnt, counters, part, M < 64, X32);
     };
     const bool small = K <= 4096;
     // the normed form keeps rms_norm_rows4_k's 256 threads and summation order
@@ -1026,7 +1048,8 @@ bool few_rows_product(float *const *Y, const void *const *W, const int *types, c
         a.Sx = Sx;
         a.Rs = Rs;
         a.R = nmat == 1 ? R : nullptr;
-        a.part = (float *)(ws + ob + sb + rb + cb);
+        a.X32 = X32;
+        a.part = (float *)(ws + ob + sb + rb + cb + xb);
         a.cnt = cnt;
         a.M = M;
         a.nb = nb;

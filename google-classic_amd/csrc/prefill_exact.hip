@@ -1572,7 +1572,7 @@ bool exact_product(float *const *Y, const void *const *W, const int *types, cons
     // one workgroup per row, K <= 16384 (exact_ok): the row in registers
     auto split = [&](auto kern, int nt) {
         hipLaunchKernelGGL(kern, dim3(M), dim3(nt), 0, stream(), (uint2 *)Ah, (uint2 *)Al, need_sx ? Sx : nullptr,
-                           Rs, X, U, NW, K, eps, nullptr, 0, 0, false);
+                           Rs, X, U, NW, K, eps, nullptr, 0, 0, false, nullptr);
     };
     // the normed form keeps rms_norm_rows4_k's 256 threads (its sum of squares
     // in the same order); the others reduce only a maximum, so their threads
