@@ -1442,9 +1442,19 @@ int exact_kind(int type)
 // (68 us on the few-row tiles, 59 on these) and 192 (104, 84) among them.
 // `full`: the launch puts both of its workgroups on every CU (above 256 rows,
 // one: 958 x 1427 x 10240 Q8_0 then takes 117, the few-row tiles 140).
+// Q4_0 and Q8_0 of an odd block count run the first tiling, 64 x 128 tiles of
+// whole K, one a CU and round: 7.75 us and a round's 0.31 a block, 30% more with
+// every CU taken (128 shapes, us there / few rows: Q4_0 192 x 11008 x 4128 106 /
+// 74, 192 x 8192 x 1056 22.6 / 24.9, 512 x 2048 x 1056 Q8_0 20.8 / 22.6).
 float exact_tiles_us(int type, int N, int M, int nb, bool prepared, bool *full)
 {
     const int ntm = (M + 63) / 64, nct = (N + 255) / 256, nst = (nb + 1) / 2;
+    if ((type == HOLO_TYPE_Q4_0 || type == HOLO_TYPE_Q8_0) && nb % 2 != 0) {
+        *full = false;
+        const int tiles = ntm * ((N + 127) / 128), rounds = tiles / num_cus(), rest = tiles % num_cus();
+        const float filled = 1.3f * (float)rounds + (rest ? 1.f + 0.3f * (float)rest / (float)num_cus() : 0.f);
+        return 7.75f + 0.31f * (float)nb * filled;
+    }
     const int gr = x2_ranges(nct, nst, ntm);
     *full = M > 256 ? ntm * gr > num_cus() : ntm * gr >= 2 * num_cus();
     const float stage = type == HOLO_TYPE_Q4_K ? 1.5f : type == HOLO_TYPE_Q6_K ? 2.0f : type == HOLO_TYPE_Q8_0 ? 1.7f : 1.25f;

@@ -15,6 +15,8 @@ MEASURED = [
     (Q6_K, 64, 14336, 4096, 1, 40, 45), (Q6_K, 80, 14336, 4096, 1, 67, 59), (Q6_K, 100, 14336, 4096, 1, 68, 59),
     (Q6_K, 192, 14336, 4096, 1, 104, 84), (Q6_K, 100, 14336, 4096, 0, 69, 86), (Q6_K, 100, 4096, 4096, 1, 28, 45),
     (Q6_K, 140, 4096, 11008, 1, 83, 90), (Q6_K, 64, 4096, 14336, 1, 46, 105), (Q6_K, 512, 14336, 4096, 1, 236, 162),
+    (Q4_0, 192, 11008, 4128, 0, 74, 106), (Q4_0, 192, 8192, 1056, 0, 25, 23), (Q8_0, 512, 2048, 1056, 0, 23, 21),
+    (Q8_0, 256, 4096, 11040, 0, 97, 125), (Q8_0, 1000, 1024, 4128, 0, 67, 57), (Q8_0, 64, 8192, 1056, 0, 12, 16),
     (Q4_0, 64, 4096, 4128, 0, 21, 50), (Q4_0, 512, 11008, 4096, 0, 240, 118)]
 
 
