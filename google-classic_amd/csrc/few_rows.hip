@@ -7,7 +7,9 @@
 // llm.c:770-926).  The arithmetic here is prefill_exact.hip's: activations as
 // two f16 halves of a row scaled by a power of two, the blocks' integers exact
 // in f16, per 32-block C = sum_k (xh + xl) * w on the f16 matrix cores, then
-// acc = fmaf(scale, C, acc) in fp32.
+// acc = fmaf(scale, C, acc) in fp32.  Rows that the halves do not hold
+// (infinities; under 64 rows also blocks far below the row's largest value) are
+// left as fp32 by the split and multiplied so at the end.
 //
 // Workgroup: 8 waves and a tile of 16 MT rows by 16 CT columns; each wave
 // multiplies the whole tile over its own eighth of K (of the workgroup's part
@@ -30,13 +32,14 @@
 // transpose over the lane groups (v_permlane32_swap, v_permlane16_swap) hands
 // every group its dword of all four blocks.
 //
-// What bounds it (512 workgroups of M = 16, 11008 x 4096): the CU's address
-// unit, three quarters busy, mostly with activation operands (4 bytes per
-// value, read once per workgroup), then the unpacking.  Measured with the
-// split launch, us, one GEMV per row -> this kernel (Q4_0, 16 rows):
-// 4096 x 4096 70.5 -> 11.9, 11008 x 4096 118.6 -> 14.9, 4096 x 11008 121.4 ->
-// 20.2; 64 rows, 64 x 256 tiles -> this kernel: 39.0 -> 16.1, 40.3 -> 24.9,
-// 73.2 -> 31.2.
+// What bounds it (16 x 11008 x 4096 Q4_0, 230 workgroups of 16 x 48): the CU's
+// address unit, 61% of a CU's time busy (TA_TA_BUSY over SQ_BUSY_CU_CYCLES),
+// mostly with activation operands (4 bytes per value, read once per workgroup),
+// beside vector instructions (44%) and products (a quarter), which two waves a
+// SIMD do not overlap.  Measured with the split launch, three matrices in turn,
+// us, one GEMV per row -> this kernel (Q4_0, 16 rows): 4096 x 4096 67.6 -> 10.8,
+// 11008 x 4096 118.9 -> 15.1, 4096 x 11008 118.6 -> 19.9; 64 rows, 64 x 256 tiles
+// -> this kernel: 38.8 -> 16.1, 39.9 -> 25.2, 72.9 -> 29.8.
 #include "common.h"
 #include "quant_blocks.h"
 #include "activation_split.h"
@@ -80,13 +83,13 @@ constexpr int kFrWaves = 8;
 // 11; three rows 13.7 against 11.4.
 constexpr int kFrMinRows = 3;
 // From 64 rows the estimates choose between this and the 64 x 256 tiles (us
-// there against here: 256 x 4096 x 4096 45.7 / 32.2, 192 x 11008 x 4096 71.4 /
-// 59.5, 512 x 1024 x 4096 44.7 / 26.5, 256 x 11008 x 4096 72.8 / 74.2), and
-// the tiles run where they fill every CU twice (512 x 4096 x 4096: 65.5 / 55.0,
-// 916 x 4082 x 2336 Q8_0: 74.7 / 119.8) or
-// this would take more than three rounds of workgroups (764 x 14319 x 1792
-// Q6_K, eleven rounds: 128 / 202: the weights leave the caches between the
-// row tiles), and above this many rows.
+// there against here: 256 x 4096 x 4096 44.6 / 33.1, 192 x 11008 x 4096 74.8 /
+// 63.7, 512 x 1024 x 4096 44.3 / 26.3, 256 x 11008 x 4096 72.1 / 77.9), and
+// the tiles run where they fill every CU twice (512 x 11008 x 4096 122 / 150, 916
+// x 4082 x 2336 Q8_0 72 / 121; the line is a coarse one: 512 x 4096 x 4096, 65.4
+// / 58.8, falls on the wrong side of it) or this would take more than three
+// rounds of workgroups (764 x 14319 x 1792 Q6_K, eleven rounds: 129 / 202: the
+// weights leave the caches between the row tiles), and above this many rows.
 constexpr int kFrMaxRows = 1024;
 constexpr int64_t kFrMaxParts = 16 << 20;  // bytes of the K parts of a launch
 constexpr int kFrMaxCounters = 4096;
@@ -810,9 +813,9 @@ constexpr int few_max_ct(int kind, int mt) { return kind == EW_F16 || (kind == E
 // per product tile; a round of workgroups over the CUs 0.75, a second part of
 // K its exchange, 3.2; and at least the activation operands of all workgroups
 // out of L2, 22.5 TB/s.  Above 32 rows 64-row tiles: more, narrower row tiles
-// read the weights again (64 x 11008 x 4096: 26.4 against 32.8).  At 16 rows
-// of 11008 x 4096: 48 columns and one round 16.0, 32 columns 18.3, 64 columns
-// 18.9, 16 columns 19.2.
+// read the weights again (64 x 11008 x 4096: 25.2 against 30.8).  At 16 rows
+// of 11008 x 4096: 48 columns and one round 15.1, 32 columns 17.4, 64 columns
+// 17.9, 16 columns 19.2.
 FrPlan few_plan(int kind, const int *N, int nmat, int M, int nb)
 {
     FrPlan best = {};
@@ -970,8 +973,8 @@ bool few_choose(const int *types, const int *N, const bool *prepared, int nmat, 
     }
     // From 64 rows on, the other tiling where it is estimated 6% better (both
     // sides measured on 70 shapes: the taken one is the faster or within 5% for
-    // all that are not `full`): 192 x 11008 x 4096 Q4_0 here 59.5 us, there 71.4;
-    // 231 x 6825 x 5632 Q6_K 92.3 and 87.1; 1015 x 890 x 4864 Q8_0 71.2 and 59.4.
+    // all that are not `full`): 192 x 11008 x 4096 Q4_0 here 63.7 us, there 74.8;
+    // 231 x 6825 x 5632 Q6_K 92.6 and 88.1; 1015 x 890 x 4864 Q8_0 70.8 and 58.4.
     return M < 64 || !(many || tiled <= 0.94f * here);
 }
 

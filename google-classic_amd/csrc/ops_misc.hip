@@ -1094,7 +1094,7 @@ bool attention_decode_fits(const float *q, const float *kc, const float *vc, int
     return hd >= 4 && hd <= 128 && hd % 4 == 0 && !(((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15);
 }
 
-// Ranges of a call: one where the whole cache fits two passes of one
+// Ranges of a call: one where the whole cache fits four passes of one
 // workgroup (256 positions of 128: 5.2 us in one launch, 7.0 in two; 400:
 // 8.2 / 7.1), else about one workgroup per CU, of at least 64 positions (1024
 // positions x 32 heads: 8 ranges 9.5 us, 4 12.1, 16 10.8), and no more than
