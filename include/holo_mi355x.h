@@ -35,7 +35,8 @@ const char *holo_error_string(int code);
  * All ops launch on one library stream (default: the null stream, as the
  * reference).  Events are recorded on that stream.  A graph captures every
  * op issued between begin and end on that stream (stream capture), so a
- * decode step of many GEMVs replays with one launch.                        */
+ * decode step of many GEMVs replays with one launch.  Scratch of captured
+ * attention and few-row calls is the graph's own until holo_graph_destroy.  */
 void holo_set_stream(void *hip_stream);
 void *holo_get_stream(void);
 void *holo_event_create(void);
@@ -226,13 +227,16 @@ int holo_prefill_get_q8_kernel(void);
 /* Y[M][N] = X[M][K] . W[N][K]^T for W in Q4_0.  3 <= M < 64 runs the exact
  * product below in tiles for few rows (in the default GEMV activation mode, K
  * <= 16384 and a multiple of 32, X 16-byte aligned; a scratch buffer per
- * stream that the library keeps, stream-ordered under capture; without memory
- * for it M GEMVs).  M >= 64 runs, by the mode set below: the exact product (HOLO_PREFILL_EXACT, the default: each row of
- * X scaled by a power of two and split into two f16 halves, x - xh - xl
- * within 2^-22 |x|, times the block's integers, exact in f16, on the f16
- * matrix cores, block scales applied in fp32 in block order; fp32 accuracy,
- * within 1e-3 of the CPU path; X 16-byte aligned and K <= 16384, else M
- * GEMVs; the tiles for few rows where they are the faster ones, else the
+ * stream that the library keeps, under capture the graph's own; without memory
+ * for it M GEMVs; a row with an infinity, or with a block of 32 values wholly
+ * below 2^-17 of its largest, is multiplied in fp32).  M >= 64 runs, by the
+ * mode set below: the exact product (HOLO_PREFILL_EXACT, the default: each row
+ * of X scaled by a power of two and split into two f16 halves, x - xh - xl
+ * within 2^-22 |x| or 2^-40 of the row's largest, times the block's integers,
+ * exact in f16, on the f16 matrix cores, block scales applied in fp32 in block
+ * order; fp32 accuracy, within 1e-3 of the CPU path; X 16-byte aligned and K
+ * <= 16384, else M GEMVs; the tiles for few rows where they are the faster
+ * ones (a row with an infinity in fp32 there too), else the
  * K blocks of each row of tiles are dealt evenly to about two
  * workgroups per CU, and a tile whose blocks two or more workgroups share
  * is the sum of their parts in K order, so the result depends on the
@@ -287,7 +291,7 @@ void holo_matmul_batch_q4_0_multi(float *const *Y, const void *const *W, const i
  * them.  Every other type, for M >= 3 and K whole blocks (Q4_K, Q6_K: K a
  * multiple of 256) up to 16384, runs the exact product by default (the block
  * integers against the two f16 halves of X, block scales in fp32; F32
- * matrices run GEMVs); in HOLO_PREFILL_F16 mode, for M >= 64, it is dequantised into an f16 panel
+ * matrices run GEMVs, and so does F16 with M < 64 and K < 1024); in HOLO_PREFILL_F16 mode, for M >= 64, it is dequantised into an f16 panel
  * (holo_dequant_f16, N*K*2 bytes per matrix) and multiplied on the f16
  * product.  Workspaces live in device buffers the library keeps and grows
  * (hipMalloc, outside graph capture; under capture a stream-ordered
