@@ -285,6 +285,7 @@ int holo_graph_begin(void)
         HOLO_REJECT("holo_graph_begin: set a non-null library stream first");
         return -1;
     }
+    holo::stream_scratch_reclaim();
     hipError_t e = hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
         holo::latch_error((int)e, "hipStreamBeginCapture", __FILE__, __LINE__);

@@ -38,5 +38,6 @@ void stream_scratch_drop(hipStream_t st);  // a stream's, before it is destroyed
 // A graph's parts of the arena, by the id of its capture: captures that end in
 // holo_graph_destroy give them back; of others they stay taken.
 void stream_scratch_drop_capture(unsigned long long id);
+void stream_scratch_reclaim();  // what a drop under an open capture left
 
 }  // namespace holo

@@ -73,10 +73,12 @@ struct Part {
     size_t at, bytes;
     unsigned long long id;
     hipStream_t stream;
+    bool dropped;  // its graph is gone
 };
 constexpr size_t kArena = (size_t)16 << 20, kMaxPart = (size_t)1 << 20;
 uint8_t *g_arena = nullptr;
 std::vector<Part> g_parts;
+bool g_dropped = false;  // some part is
 
 // At least `bytes` for capture `id` on the library stream; nullptr when they
 // do not fit.  g_mu is held.
@@ -90,8 +92,22 @@ void *arena_part(size_t bytes, unsigned long long id)
     auto it = g_parts.begin();
     for (; it != g_parts.end() && it->at - at < bytes; ++it) at = it->at + it->bytes;
     if (at + bytes > kArena) return nullptr;
-    g_parts.insert(it, Part{at, bytes, id, stream()});
+    g_parts.insert(it, Part{at, bytes, id, stream(), false});
     return g_arena + at;
+}
+
+// Gives the dropped parts back, once the device is idle: a last replay may be
+// under way.  Not while a capture is open, which waiting would end: the next
+// holo_graph_begin or _destroy does it then.  g_mu is held.
+void reclaim()
+{
+    if (!g_dropped || stream_capturing()) return;
+    if (hipDeviceSynchronize() != hipSuccess) {  // another thread captures
+        (void)hipGetLastError();
+        return;
+    }
+    g_parts.erase(std::remove_if(g_parts.begin(), g_parts.end(), [](const Part &p) { return p.dropped; }), g_parts.end());
+    g_dropped = false;
 }
 
 }  // namespace
@@ -133,14 +149,15 @@ bool stream_scratch_init()
 void stream_scratch_drop_capture(unsigned long long id)
 {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (std::none_of(g_parts.begin(), g_parts.end(), [&](const Part &p) { return p.id == id; })) return;
-    // the graph's last replay may be under way
-    if (hipDeviceSynchronize() != hipSuccess) {  // another thread captures: they stay taken
-        (void)hipGetLastError();
-        return;
-    }
-    g_parts.erase(std::remove_if(g_parts.begin(), g_parts.end(), [&](const Part &p) { return p.id == id; }),
-                  g_parts.end());
+    for (Part &p : g_parts)
+        if (p.id == id) p.dropped = g_dropped = true;
+    reclaim();
+}
+
+void stream_scratch_reclaim()
+{
+    std::lock_guard<std::mutex> lk(g_mu);
+    reclaim();
 }
 
 void stream_scratch_release()
@@ -149,6 +166,7 @@ void stream_scratch_release()
     if (g_arena) (void)hipFree(g_arena);
     g_arena = nullptr;
     g_parts.clear();
+    g_dropped = false;
     for (Slot &s : g_slots) {
         if (s.buf) (void)hipFree(s.buf);
         s = Slot{};

@@ -208,7 +208,19 @@ def test_decode_graphs_own_their_partials(holo, synth):
             for g, _ in graphs:
                 lib.holo_graph_launch(g)
             lib.cuda_sync()
-            for i, (g, d) in enumerate(graphs):
+            # a graph destroyed while another is captured does not disturb it
+            spare, old, d = graphs.pop(), graphs.pop(0), holo.DeviceBuffer(4 * nh * hd)
+            assert lib.holo_graph_begin() == 0
+            lib.holo_graph_destroy(old[0])
+            lib.cuda_multi_head_attention(d.ptr, qs[1].ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+            graphs.insert(0, (lib.holo_graph_end(), d))
+            holo.check("capture beside a destroy")
+            lib.holo_graph_launch(graphs[0][0])
+            lib.holo_graph_destroy(spare[0])
+            lib.cuda_sync()
+            assert np.array_equal(down(d, nh * hd).view(np.uint32), want[1]), turn
+            lib.holo_graph_destroy(graphs.pop(0)[0])
+            for i, (g, d) in enumerate(graphs, 1):
                 assert np.array_equal(down(d, nh * hd).view(np.uint32), want[i % 4]), (turn, i)
                 lib.holo_graph_destroy(g)
     finally:
