@@ -108,7 +108,7 @@ int cuda_init(void)
         return -1;
     }
     if (!holo::stream_scratch_init()) {
-        fprintf(stderr, "holo_mi355x: cannot allocate the captured calls' scratch\n");
+        fprintf(stderr, "holo_mi355x: cannot allocate the calls' scratch\n");
         return -1;
     }
     if (!holo::exact_init()) {

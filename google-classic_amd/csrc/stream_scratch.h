@@ -8,14 +8,16 @@
 namespace holo {
 
 // Scratch for the launches of one call, from its construction to its
-// destruction, in stream order.  One kept buffer per stream, so calls on
-// several streams never share one, for up to 8 streams; a further stream takes
-// over the least recently used buffer once the device is idle.  The pool's lock
+// destruction, in stream order.  Kept per stream, so calls on several streams
+// never share it: up to 512 KiB a part of an arena that cuda_init allocates (so
+// a decode attention allocates nothing, also while another stream is captured),
+// above that a buffer, for up to 8 streams; a further stream takes over the
+// least recently used buffer once the device is idle.  The pool's lock
 // is held meanwhile, so calls of several threads on one stream run one after
 // the other.  (Stream-ordered allocations instead cost about 10 us of host time
-// a call.)  Under capture a part of the capture arena that is the graph's own (a
-// graph must not hold a kept buffer, which eager calls on its stream use too
-// and another stream may take over), or, past 1 MiB or with the arena full, a
+// a call.)  Under capture a part of the arena that is the graph's own (a
+// graph must not hold the stream's scratch, which eager calls use too and
+// another stream may take over), or, past 1 MiB or with the arena full, a
 // stream-ordered allocation (whose nodes cost a replay about 15 us a call: 32
 // decode attentions at 600 positions 196 us, with them 673).
 class StreamScratch {
@@ -32,7 +34,7 @@ private:
     bool free_ = false;  // a stream-ordered allocation
 };
 
-bool stream_scratch_init();  // the capture arena
+bool stream_scratch_init();  // the arena
 void stream_scratch_release();  // all of it
 void stream_scratch_drop(hipStream_t st);  // a stream's, before it is destroyed
 // A graph's parts of the arena, by the id of its capture: captures that end in

@@ -67,20 +67,20 @@ void *slot(size_t bytes)
     return s->buf;
 }
 
-// The capture arena's parts in order of address.  The calls of one capture on
-// one stream run in order and share a part.
+// The arena's parts in order of address.  The calls of one capture on one stream
+// run in order and share a part, and so do the small eager calls of a stream.
 struct Part {
     size_t at, bytes;
-    unsigned long long id;
+    unsigned long long id;  // of the capture; 0: eager calls
     hipStream_t stream;
     bool dropped;  // its graph is gone
 };
-constexpr size_t kArena = (size_t)16 << 20, kMaxPart = (size_t)1 << 20;
+constexpr size_t kArena = (size_t)16 << 20, kMaxPart = (size_t)1 << 20, kSmallPart = (size_t)512 << 10;
 uint8_t *g_arena = nullptr;
 std::vector<Part> g_parts;
 bool g_dropped = false;  // some part is
 
-// At least `bytes` for capture `id` on the library stream; nullptr when they
+// At least `bytes` for capture `id` (or eager calls) on the library stream; nullptr when they
 // do not fit.  g_mu is held.
 void *arena_part(size_t bytes, unsigned long long id)
 {
@@ -121,7 +121,7 @@ StreamScratch::StreamScratch(size_t bytes) : lock_(g_mu)
         return;
     }
     if (st == hipStreamCaptureStatusNone) {
-        buf_ = slot(bytes);
+        if (bytes > kSmallPart || (buf_ = arena_part(bytes, 0)) == nullptr) buf_ = slot(bytes);
     } else if ((buf_ = arena_part(bytes, id)) == nullptr) {
         free_ = hipMallocAsync(&buf_, bytes, stream()) == hipSuccess;
         if (!free_) {
@@ -182,6 +182,11 @@ void stream_scratch_drop(hipStream_t st)
             if (s.buf) (void)hipFree(s.buf);
             s = Slot{};
         }
+    auto small = [&](const Part &p) { return p.id == 0 && p.stream == st; };
+    if (std::any_of(g_parts.begin(), g_parts.end(), small)) {
+        (void)hipStreamSynchronize(st);
+        g_parts.erase(std::remove_if(g_parts.begin(), g_parts.end(), small), g_parts.end());
+    }
 }
 
 }  // namespace holo

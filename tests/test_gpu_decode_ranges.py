@@ -182,6 +182,43 @@ def test_decode_streams_and_graph(holo, synth, kv_len):
     holo.check("streams")
 
 
+def test_decode_on_one_stream_while_another_is_captured(holo, synth):
+    """An eager call of several ranges, the first on its stream, allocates
+    nothing, so it may run while the thread captures another stream."""
+    lib = holo.lib()
+    hd, nh, nkv, kv_len = 128, 32, 8, 600
+    kc, vc = (up(holo, synth.normal(kv_len * nkv * hd, seed=98 + i)) for i in range(2))
+    q = up(holo, synth.normal(nh * hd, seed=100))
+    outs = [holo.DeviceBuffer(4 * nh * hd) for _ in range(3)]
+
+    def call(d):
+        lib.cuda_multi_head_attention(d.ptr, q.ptr, kc.ptr, vc.ptr, kv_len, hd, nh, nkv)
+
+    call(outs[0])
+    lib.cuda_sync()
+    want = down(outs[0], nh * hd).view(np.uint32)
+    a, b = lib.holo_stream_create(), lib.holo_stream_create()
+    try:
+        lib.holo_set_stream(a)
+        assert lib.holo_graph_begin() == 0
+        call(outs[1])
+        lib.holo_set_stream(b)
+        call(outs[2])
+        lib.holo_set_stream(a)
+        g = lib.holo_graph_end()
+        holo.check("capture beside an eager call")
+        lib.holo_graph_launch(g)
+        lib.cuda_sync()
+        for d in outs[1:]:
+            assert np.array_equal(down(d, nh * hd).view(np.uint32), want)
+        lib.holo_graph_destroy(g)
+    finally:
+        lib.holo_set_stream(None)
+        lib.holo_stream_destroy(a)
+        lib.holo_stream_destroy(b)
+    holo.check("streams")
+
+
 def test_decode_graphs_own_their_partials(holo, synth):
     """More captured graphs alive than the library's capture scratch holds, and
     again after they are gone: every replay gives the eager call's bits."""
